@@ -29,8 +29,9 @@ Plan *build_batch_plan(Ctx *ctx, int64_t n, Plan *const *members) {
   p->precision = QLG_PREC_F64;
   p->nphys = members[0]->nphys;
   // arena bases of every member, per slot
-  std::vector<std::array<int64_t, NSLOTS>> base(n);
+  std::vector<std::array<int64_t, NSLOTS>> base(n), rbase(n);
   int64_t vs = 0, xs = 0, ys = 0, cs = 0, ls = 0, rs = 0;
+  int64_t yrs = 0, lrs = 0, rrs = 0;   // reduced form
   p->batch_off.assign(n + 1, 0);
   for (int64_t m = 0; m < n; ++m) {
     const Plan &q = *members[m];
@@ -42,6 +43,23 @@ Plan *build_batch_plan(Ctx *ctx, int64_t n, Plan *const *members) {
     b[SLOT_C] = cs;
     b[SLOT_L] = ls;
     b[SLOT_R] = rs;
+    rbase[m] = b;
+    rbase[m][SLOT_Y] = yrs;
+    rbase[m][SLOT_L] = lrs;
+    rbase[m][SLOT_R] = rrs;
+    for (TransDesc c : q.red_l) {
+      c.src += ls;
+      c.dst += lrs;
+      p->red_l.push_back(c);
+    }
+    for (TransDesc c : q.red_r) {
+      c.src += rs;
+      c.dst += rrs;
+      p->red_r.push_back(c);
+    }
+    yrs += q.yred_elems;
+    lrs += q.lred_elems;
+    rrs += q.rred_elems;
     vs += q.vec.size;
     xs += q.x_elems;
     ys += q.y_elems;
@@ -59,12 +77,16 @@ Plan *build_batch_plan(Ctx *ctx, int64_t n, Plan *const *members) {
   p->c_elems = cs;
   p->lint_elems = ls;
   p->rint_elems = rs;
-  // task lists
-  for (int i = 0; i < 3; ++i) {
-    Stage &d = p->st[i];
+  p->yred_elems = yrs;
+  p->lred_elems = lrs;
+  p->rred_elems = rrs;
+  // task lists, in both forms
+  for (int i = 0; i < 6; ++i) {
+    const bool red = i >= 3;
+    Stage &d = red ? p->rst[i - 3] : p->st[i];
     for (int64_t m = 0; m < n; ++m) {
-      const Stage &s = members[m]->st[i];
-      const auto &b = base[m];
+      const Stage &s = red ? members[m]->rst[i - 3] : members[m]->st[i];
+      const auto &b = red ? rbase[m] : base[m];
       const int32_t seg0 = (int32_t)d.segs.size(), crow0 = (int32_t)d.crows.size();
       for (GemmSeg g : s.segs) {
         g.a_off += b[g.a_slot];
@@ -117,14 +139,18 @@ Plan *build_batch_plan(Ctx *ctx, int64_t n, Plan *const *members) {
   }
   int64_t slot_elems[NSLOTS] = {0, vs, vs, ls, rs, xs, ys, cs};
   for (int i = 0; i < 3; ++i) validate_stage(p->st[i], slot_elems);
+  int64_t red_elems[NSLOTS] = {0, vs, vs, lrs, rrs, xs, yrs, cs};
+  for (int i = 0; i < 3; ++i) validate_stage(p->rst[i], red_elems);
+  p->st[0].find_direct();
+  p->st[2].find_direct();
   // arenas: operators copied from the members, intermediates fresh
   hipStream_t st = ctx->stream;
   const size_t eb = sizeof(double);
   p->X.ensure(std::max<int64_t>(xs, 1) * eb);
-  p->Y.ensure(std::max<int64_t>(ys, 1) * eb);
+  p->Y.ensure((ys + 2) * eb);
   p->C.ensure(std::max<int64_t>(cs, 1) * eb);
-  p->Lint.ensure(std::max<int64_t>(ls, 1) * eb);
-  p->Rint.ensure(std::max<int64_t>(rs, 1) * eb);
+  p->Lint.ensure((ls + 2) * eb);
+  p->Rint.ensure((rs + 2) * eb);
   QLG_HIP(hipMemsetAsync(p->Y.p, 0, std::max<int64_t>(ys, 1) * eb, st));   // Y entries no channel writes stay zero
   for (int64_t m = 0; m < n; ++m) {
     const Plan &q = *members[m];
@@ -146,13 +172,7 @@ Plan *build_batch_plan(Ctx *ctx, int64_t n, Plan *const *members) {
     QLG_HIP(hipMemcpyAsync(p->d_pack_out.p, p->pack_out.data(), p->pack_out.size() * sizeof(CopyDesc),
                            hipMemcpyHostToDevice, st));
   }
-  for (int i = 0; i < 3; ++i) {
-    if (i == 1)
-      p->st[i].make_tiles(members[0]->st[1].bm, members[0]->st[1].bn);
-    else
-      model_tiles(p->st[i], false);   // replaced by measured shapes on the first matvec
-    p->st[i].upload(st);
-  }
+  p->prepare_lists();
   p->st[0].algo_bytes = 8.0 * double(ls + vs + xs);
   p->st[1].algo_bytes = 8.0 * double(xs + cs + ys);
   p->st[2].algo_bytes = 8.0 * double(ys + rs + vs);

@@ -295,6 +295,266 @@ static void launch_shape(int bm, int bn, int bk, const GemmTile *tiles, const Ge
   throw Error(QLG_ERR_UNSUPPORTED, "unsupported FP64 tile shape");
 }
 
+// ---------------------------------------------------------------------------
+// FP64 GEMM with operand fragments loaded straight from memory (the matvec's
+// two contractions): C = A^T B with A stored [K x M] and B stored [K x N].
+//
+// A v_mfma_f64_16x16x4 takes 64 cycles, so a wave's matrix pipe is fed by few
+// bytes per cycle: what bounds the matvec's tasks is the latency of the
+// operand loads.  A lane loads exactly the operand values its MFMAs take,
+// kDepth slices ahead, in registers: no LDS, no barrier, no per-element
+// address arithmetic (the k offset of a slice is the load's scalar offset).
+// Both operands are stored with k as the row index, so that the sixteen lanes
+// that share a k read one contiguous run: with k contiguous the same lanes
+// touch sixteen cache lines per load.
+//
+// Real data: two 16-wide blocks of a wave's tile are interleaved (lane l holds
+// elements 2 (l % 16) and 2 (l % 16) + 1 of 32), so one 16-byte load feeds both.
+// Such a load may reach one element past an odd-width operand's last column;
+// the value lands in a row or column that is never stored, and the vectors'
+// buffers carry that one element of slack.
+//
+// A workgroup's waves are WM x WN over the tile and WK over k: k-part w takes
+// slices w, w + WK, ...; the parts are summed through LDS in order at the end.
+// Small tiles use WK > 1, so that long-K tasks with few columns keep every
+// SIMD busy.
+// ---------------------------------------------------------------------------
+__device__ inline double2 load_pair(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+  typedef double d2 __attribute__((ext_vector_type(2)));
+  const d2 v = __builtin_bit_cast(d2, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+  return double2{v.x, v.y};
+}
+
+// position within the wave's tile of block i's element c (c < 16)
+template <int F, bool CPLX>
+__device__ inline int frag_pos(int i, int c) {
+  if constexpr (CPLX || F % 2) return i * 16 + c;
+  return (i / 2) * 32 + 2 * c + (i & 1);
+}
+
+// Fragments of F 16-wide blocks of one operand over a slice of KD rows;
+// step t multiplies row k0 + 4 t + lane / 16.
+template <int F, int KD, bool CPLX>
+struct FragLoader {
+  static constexpr bool PAIR = !CPLX && F % 2 == 0;
+  static constexpr int NL = PAIR ? F / 2 : F;          // loads per k-step
+  static constexpr uint32_t EB = CPLX ? 16u : 8u;
+  struct Frag {
+    double v[F][KD / 4][CPLX ? 2 : 1];
+  };
+  __amdgpu_buffer_rsrc_t rs;
+  uint32_t off[NL];      // byte offset of the lane's element in slice 0, or kOob
+  uint32_t kstep;        // bytes from row k to k + 1
+  int kq, K;
+  __device__ void setup(const void *base, int64_t ld, int Kseg, int x0, int X, int lane) {
+    rs = make_rsrc(base);
+    K = Kseg;
+    kq = lane >> 4;
+    kstep = (uint32_t)ld * EB;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int x = x0 + frag_pos<F, CPLX>(PAIR ? 2 * i : i, lane & 15);
+      off[i] = x < X ? (uint32_t)kq * kstep + (uint32_t)x * EB : kOob;
+    }
+  }
+  // loads past K return zeros without touching memory
+  __device__ void load(Frag &f, int k0) const {
+    const uint32_t s0 = k0 < K ? (uint32_t)k0 * kstep : 0u;   // masked loads keep a small scalar offset
+#pragma unroll
+    for (int t = 0; t < KD / 4; ++t) {
+      const bool ok = k0 + 4 * t + kq < K;
+#pragma unroll
+      for (int i = 0; i < NL; ++i) {
+        const uint32_t o = ok ? off[i] : kOob, so = s0 + 4u * t * kstep;
+        if constexpr (CPLX) {
+          const double2 x = load_pair(rs, o, so);
+          f.v[i][t][0] = x.x;
+          f.v[i][t][1] = x.y;
+        } else if constexpr (PAIR) {
+          const double2 x = load_pair(rs, o, so);
+          f.v[2 * i][t][0] = x.x;
+          f.v[2 * i + 1][t][0] = x.y;
+        } else {
+          f.v[i][t][0] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, o, so, 0));
+        }
+      }
+    }
+  }
+};
+
+template <int FM, int FN, int WM, int WN, int WK, int kDepth, bool CPLX>
+__global__ __launch_bounds__(64 * WM * WN * WK, FM * FN * (CPLX ? 2 : 1) <= 8 ? 2 : 1) void direct_gemm_f64_kernel(const GemmTile *__restrict__ tiles,
+                                                                            const GemmTask *__restrict__ tasks,
+                                                                            const GemmSeg *__restrict__ segs,
+                                                                            Slots slots, int ntiles) {
+  constexpr int KD = CPLX ? 8 : 16;
+  constexpr int NP = CPLX ? 2 : 1;
+  using LA = FragLoader<FM, KD, CPLX>;
+  using LB = FragLoader<FN, KD, CPLX>;
+  if ((int)blockIdx.x >= ntiles) return;
+  if (slots.skip && *slots.skip) return;   // the Krylov solve has stopped
+  const GemmTile tl = tiles[blockIdx.x];
+  if (tl.task < 0) return;  // padding slot of the XCD-balanced launch order
+  const GemmTask tk = tasks[tl.task];
+  const int M = tk.M, N = tk.N;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wk = wave / (WM * WN), wmn = wave % (WM * WN);
+  const int m0 = tl.m0 + (wmn / WN) * FM * 16, n0 = tl.n0 + (wmn % WN) * FN * 16;
+
+  dbl4 acc[NP][FM][FN];
+#pragma unroll
+  for (int p = 0; p < NP; ++p)
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[p][i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+
+  typename LA::Frag fa[kDepth];
+  typename LB::Frag fb[kDepth];
+  for (int s = tk.seg_begin; s < tk.seg_begin + tk.seg_count; ++s) {
+    const GemmSeg sg = segs[s];
+    const int K = sg.K;
+    if (K <= 0) continue;
+    LA la;
+    LB lb;
+    la.setup(slots.p[sg.a_slot] + sg.a_off * NP, sg.lda, K, m0, M, lane);
+    lb.setup(slots.p[sg.b_slot] + sg.b_off * NP, sg.ldb, K, n0, N, lane);
+    const int ns = ((K + KD - 1) / KD - wk + WK - 1) / WK;   // this wave's slices
+    auto fetch = [&](int d, int n) {
+      la.load(fa[d], (n * WK + wk) * KD);
+      lb.load(fb[d], (n * WK + wk) * KD);
+      // keep the slices' loads in order: the wait before a slice's MFMAs then
+      // leaves the later slices' loads in flight
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](int d) {
+#pragma unroll
+      for (int t = 0; t < KD / 4; ++t)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) {
+            const double *a = fa[d].v[i][t], *b = fb[d].v[j][t];
+            acc[0][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0], b[0], acc[0][i][j], 0, 0, 0);
+            if constexpr (CPLX) {
+              acc[0][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[1], b[1], acc[0][i][j], 0, 0, 0);
+              acc[1][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0], b[1], acc[1][i][j], 0, 0, 0);
+              acc[1][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[1], b[0], acc[1][i][j], 0, 0, 0);
+            }
+          }
+    };
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d) fetch(d, d);
+    int n = 0;
+    // straight-line rounds of kDepth slices (an exit inside the round would
+    // make the compiler wait for every load at its top), then the rest
+    for (; n + 2 * kDepth <= ns; n += kDepth)
+#pragma unroll
+      for (int d = 0; d < kDepth; ++d) {
+        multiply(d);
+        fetch(d, n + d + kDepth);
+      }
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d) {
+      if (n + d < ns) multiply(d);
+      if (n + d + kDepth < ns) fetch(d, n + d + kDepth);
+    }
+#pragma unroll
+    for (int d = 0; d < kDepth - 1; ++d)
+      if (n + d + kDepth < ns) multiply(d);
+  }
+
+  if constexpr (WK > 1) {   // sum the k parts, in order
+    constexpr int R = NP * FM * FN * 4;
+    __shared__ double red[(WK - 1) * WM * WN][R][64];
+    if (wk > 0) {
+      const int w = (wk - 1) * WM * WN + wmn;
+#pragma unroll
+      for (int r = 0; r < R; ++r) red[w][r][lane] = acc[r / (FM * FN * 4)][r / (FN * 4) % FM][r / 4 % FN][r % 4];
+    }
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll 1
+    for (int q = 0; q < WK - 1; ++q)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        acc[r / (FM * FN * 4)][r / (FN * 4) % FM][r / 4 % FN][r % 4] += red[q * WM * WN + wmn][r][lane];
+  }
+
+  // output row addresses: a row-address table or a plain row stride
+  int64_t crow[FM][4];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = m0 + frag_pos<FM, CPLX>(i, (lane >> 4) + 4 * r);
+      crow[i][r] = tk.c_rowtab ? slots.crows[tk.c_row + min(row, M - 1)] : tk.c_off + (int64_t)row * tk.ldc;
+    }
+  double *C = slots.p[tk.c_slot];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = m0 + frag_pos<FM, CPLX>(i, (lane >> 4) + 4 * r);
+      if (row >= M) continue;
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const int col = n0 + frag_pos<FN, CPLX>(j, lane & 15);
+        const int64_t ix = crow[i][r] + col;
+        if constexpr (CPLX) {
+          if (col < N) reinterpret_cast<double2 *>(C)[ix] = double2{acc[0][i][j][r], acc[1][i][j][r]};
+        } else if constexpr (FN % 2 == 0) {   // blocks j, j + 1 hold neighbouring columns
+          if (j & 1) continue;
+          typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+          if (col + 1 < N)
+            *reinterpret_cast<d2u *>(C + ix) = d2u{acc[0][i][j][r], acc[0][i][j + 1][r]};
+          else if (col < N)
+            C[ix] = acc[0][i][j][r];
+        } else {
+          if (col < N) C[ix] = acc[0][i][j][r];
+        }
+      }
+    }
+}
+
+template <bool CPLX>
+static void launch_direct(int bm, int bn, const GemmTile *tiles, const GemmTask *tasks, const GemmSeg *segs,
+                          const Slots &slots, int ntiles, hipStream_t st) {
+#define QLG_DIRECT(FM_, FN_, WM_, WN_, WK_, D_)                                                               \
+  if (bm == FM_ * 16 * WM_ && bn == FN_ * 16 * WN_) {                                                         \
+    hipLaunchKernelGGL((direct_gemm_f64_kernel<FM_, FN_, WM_, WN_, WK_, D_, CPLX>), dim3(ntiles),         \
+                       dim3(64 * WM_ * WN_ * WK_), 0, st, tiles, tasks, segs, slots, ntiles);                 \
+    return;                                                                                                   \
+  }
+  if constexpr (CPLX) {
+    QLG_DIRECT(2, 2, 1, 1, 4, 2)
+    QLG_DIRECT(2, 2, 2, 1, 2, 2)
+    QLG_DIRECT(2, 2, 1, 2, 2, 2)
+    QLG_DIRECT(2, 2, 2, 2, 1, 2)
+  } else {
+    QLG_DIRECT(2, 2, 1, 1, 4, 2)
+    QLG_DIRECT(2, 2, 2, 1, 2, 3)
+    QLG_DIRECT(2, 2, 1, 2, 2, 3)
+    QLG_DIRECT(2, 2, 2, 2, 1, 3)
+    QLG_DIRECT(4, 2, 2, 2, 1, 2)
+    QLG_DIRECT(2, 4, 2, 2, 1, 2)
+    QLG_DIRECT(4, 4, 2, 2, 1, 2)
+    QLG_DIRECT(4, 1, 1, 1, 4, 2)
+    QLG_DIRECT(4, 1, 2, 1, 2, 2)
+  }
+#undef QLG_DIRECT
+  throw Error(QLG_ERR_UNSUPPORTED, "unsupported FP64 tile shape");
+}
+
+void launch_direct_gemm_f64(int bm, int bn, bool cplx, const GemmTile *tiles, const GemmTask *tasks,
+                            const GemmSeg *segs, const Slots &slots, int ntiles, hipStream_t st) {
+  if (ntiles <= 0) return;
+  cplx ? launch_direct<true>(bm, bn, tiles, tasks, segs, slots, ntiles, st)
+       : launch_direct<false>(bm, bn, tiles, tasks, segs, slots, ntiles, st);
+  QLG_HIP(hipGetLastError());
+}
+
 // Split-K reduction: every thread sums up to four elements of one task's
 // partial panels in part order and writes them where the task's epilogue
 // would (row table or row stride).

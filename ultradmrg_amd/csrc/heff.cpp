@@ -2,14 +2,16 @@
 //
 // The sector pairing is done once per plan and turned into three launches:
 //  stage 1  per ket sector a of the state:  T1_a = L_a . Psi_a, where L_a stacks
-//           every L block (a', w, a) (rows (a', w)) and Psi_a is the state's
-//           fused matrix [D_a x N_a] (all blocks (a, s1, s2, b) side by side);
+//           every L block (a', w, a) and Psi_a is the state's fused matrix
+//           [D_a x N_a] (all blocks (a, s1, s2, b) side by side);
 //  stage 2  per channel (a'-sector, b-sector): Y = C . X on rows gathered from
 //           T1 (one per (w, s1, s2) component) and scattered into Y, C being the
 //           combined MPO operator sum_y Wl[w,s1,t1,y] Wr[y,s2,t2,z];
 //  stage 3  per bra sector b': out = Y_b' . R_b'^T, where R_b' holds every R
 //           block (b', z, b) side by side (one long K) and Y_b' the rows of all
 //           output blocks with bra b'; output rows land in the fused layout.
+// The lists are made in two forms (plan.h): FP64 with k as the row index of
+// every contraction operand, the reduced modes with k contiguous.
 // The Krylov vectors inside the library use the fused layout; the boundary
 // keeps the canonical one (pack / unpack copies at the solver's entry / exit).
 #include <algorithm>
@@ -22,6 +24,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <unordered_map>
 #include <set>
 
@@ -292,38 +295,58 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
 
   pt.mark("layout");
   // ---- L stacks (ket-major) and stage 1 --------------------------------------------
+  // Reduced form: rows (a', w) of D_a elements, block after block; the leading
+  // dimension is a multiple of 8 (zero padding past K in every row): the
+  // split-BF16 kernels stage their bf16 piece planes in aligned 16-byte chunks
+  // of 8 k values.  FP64 form: D_a rows of the same stack's elements ordered
+  // (block, w, a'), so that a' runs are contiguous in T1; the leading dimension
+  // is a multiple of 16, so that a 16-wide fragment is one cache line.
   struct LStack {
-    int64_t base = 0, rows = 0;
-    std::map<int64_t, int64_t> roff;   // L block -> first row in the stack
+    int64_t base = 0, rows = 0;          // reduced form
+    int64_t kbase = 0, kld = 0;          // FP64 form
+    std::map<int64_t, int64_t> roff;     // L block -> first row (column) in the stack
   };
   std::map<int, LStack> lst;
-  std::vector<CopyDesc> lcopy;
-  int64_t lint_elems = 0;
-  // Stacks, R panels and Y panels keep a leading dimension that is a multiple
-  // of 8 (zero padding past K in every row): the split-BF16 kernels stage
-  // their bf16 piece planes in aligned 16-byte chunks of 8 k values.
+  std::vector<TransDesc> lcopy, rcopy;   // environment blocks -> FP64 form
+  int64_t lint_elems = 0, lred_elems = 0;
   auto ld8 = [](int64_t k) { return (k + 7) / 8 * 8; };
+  // (unpadded where the padding alone would push an operand past the kernels' span)
+  auto ld16 = [](int64_t x, int64_t k) {
+    const int64_t l = (x + 15) / 16 * 16;
+    return k * l * 16 < (int64_t(1) << 31) ? l : x;
+  };
   int64_t lint_alg = 0, rint_alg = 0, y_alg = 0;   // elements without the padding
   for (auto &kv : L_by_ket) {
     const int a = kv.first;
     if (!fz.count(a)) continue;
     const int64_t Da = L.ax[2].deg[a], lda = ld8(Da);
     LStack s;
-    s.base = lint_elems;
+    s.base = lred_elems;
+    s.kbase = lint_elems;
     for (int64_t lb : kv.second) {
-      const int64_t r = L.ax[0].deg[L.blk[lb][0]] * L.ax[1].deg[L.blk[lb][1]];
       s.roff[lb] = s.rows;
-      lcopy.push_back(CopyDesc{L.off[lb], s.base + s.rows * lda, Da, lda, (int32_t)r, (int32_t)Da});
-      s.rows += r;
+      s.rows += L.ax[0].deg[L.blk[lb][0]] * L.ax[1].deg[L.blk[lb][1]];
     }
-    lint_elems += s.rows * lda;
+    s.kld = ld16(s.rows, Da);
+    for (int64_t lb : kv.second) {
+      const int64_t Dap = L.ax[0].deg[L.blk[lb][0]], Wm = L.ax[1].deg[L.blk[lb][1]], r0 = s.roff[lb];
+      for (int64_t w = 0; w < Wm; ++w) {
+        const int64_t k0 = s.kbase + r0 + w * Dap;
+        lcopy.push_back(TransDesc{L.off[lb] + w * Da, k0, Wm * Da, s.kld, (int32_t)Dap, (int32_t)Da});
+        p.red_l.push_back(TransDesc{k0, s.base + (r0 + w) * lda, s.kld, Wm * lda, (int32_t)Da, (int32_t)Dap});
+      }
+    }
+    lred_elems += s.rows * lda;
+    lint_elems += Da * s.kld;
     lint_alg += s.rows * Da;
     lst[a] = s;
   }
   Stage &s1 = p.st[0], &s2 = p.st[1], &s3 = p.st[2];
-  s3.splitk = true;   // one long-K task per bra sector: split-K parts may be tuned in
-  s3.split_on = std::getenv("QLG_SPLITK") != nullptr;
-  s3.ed = ed;
+  Stage &r1 = p.rst[0], &r2 = p.rst[1], &r3 = p.rst[2];
+  // one long-K task per bra sector: split-K parts may be tuned in
+  s3.splitk = r3.splitk = true;
+  s3.split_on = r3.split_on = std::getenv("QLG_SPLITK") != nullptr;
+  s1.ed = s3.ed = r1.ed = r3.ed = ed;
   std::map<int, int64_t> tbase;
   {
     int64_t t1 = 0;
@@ -333,23 +356,36 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
       const int64_t Da = L.ax[2].deg[a], N = fz[a].N;
       tbase[a] = t1;
       GemmSeg g{};
+      g.a_slot = SLOT_IN;
+      g.a_off = fz[a].base;
+      g.lda = N;
+      g.b_slot = SLOT_L;
+      g.b_off = s.kbase;
+      g.ldb = s.kld;
+      g.K = (int32_t)Da;
+      g.flags = SEG_TRANS_A;
+      GemmTask t{};
+      t.c_slot = SLOT_X;
+      t.c_off = t1;
+      t.ldc = s.rows;
+      t.M = (int32_t)N;
+      t.N = (int32_t)s.rows;
+      t.seg_begin = (int32_t)s1.segs.size();
+      t.seg_count = 1;
+      s1.segs.push_back(g);
+      s1.tasks.push_back(t);
       g.a_slot = SLOT_L;
       g.a_off = s.base;
       g.lda = ld8(Da);
       g.b_slot = SLOT_IN;
       g.b_off = fz[a].base;
       g.ldb = N;
-      g.K = (int32_t)Da;
-      GemmTask t{};
-      t.c_slot = SLOT_X;
-      t.c_off = t1;
+      g.flags = 0;
       t.ldc = N;
       t.M = (int32_t)s.rows;
       t.N = (int32_t)N;
-      t.seg_begin = (int32_t)s1.segs.size();
-      t.seg_count = 1;
-      s1.segs.push_back(g);
-      s1.tasks.push_back(t);
+      r1.segs.push_back(g);
+      r1.tasks.push_back(t);
       s1.flops += fl * double(s.rows) * double(N) * double(Da);
       t1 += s.rows * N;
     }
@@ -359,28 +395,32 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
   pt.mark("stage1");
   // ---- R panels (bra-major) ------------------------------------------------------------
   struct RPanel {
-    int64_t base = 0, K = 0, ld = 0;
-    std::map<std::pair<int, int>, int64_t> col;   // (z sector, b sector) -> column offset
+    int64_t base = 0, K = 0, ld = 0;      // reduced form: [D_b' x K]
+    int64_t kbase = 0, kld = 0;           // FP64 form: [K x D_b']
+    std::map<std::pair<int, int>, int64_t> col;   // (z sector, b sector) -> first k
   };
   std::map<int, RPanel> rpn;
-  std::vector<CopyDesc> rcopy;
-  int64_t rint_elems = 0;
+  int64_t rint_elems = 0, rred_elems = 0;
   for (auto &kv : R_by_bra) {
     const int bp = kv.first;
     RPanel P;
-    P.base = rint_elems;
+    P.base = rred_elems;
+    P.kbase = rint_elems;
     for (int64_t rb : kv.second) {
       P.col[{R.blk[rb][1], R.blk[rb][2]}] = P.K;
       P.K += R.ax[1].deg[R.blk[rb][1]] * R.ax[2].deg[R.blk[rb][2]];
     }
     const int64_t Dbp = R.ax[0].deg[bp];
     P.ld = ld8(P.K);
+    P.kld = ld16(Dbp, P.K);
     for (int64_t rb : kv.second) {
       const int64_t w = R.ax[1].deg[R.blk[rb][1]] * R.ax[2].deg[R.blk[rb][2]];
-      rcopy.push_back(CopyDesc{R.off[rb], P.base + P.col[{R.blk[rb][1], R.blk[rb][2]}], w, P.ld, (int32_t)Dbp,
-                               (int32_t)w});
+      const int64_t c0 = P.col[{R.blk[rb][1], R.blk[rb][2]}], k0 = P.kbase + c0 * P.kld;
+      rcopy.push_back(TransDesc{R.off[rb], k0, w, P.kld, (int32_t)Dbp, (int32_t)w});
+      p.red_r.push_back(TransDesc{k0, P.base + c0, P.kld, P.ld, (int32_t)w, (int32_t)Dbp});
     }
-    rint_elems += Dbp * P.ld;
+    rred_elems += Dbp * P.ld;
+    rint_elems += P.K * P.kld;
     rint_alg += Dbp * P.K;
     rpn[bp] = P;
   }
@@ -388,7 +428,8 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
   pt.mark("rpanels");
   // ---- Y panels (per bra sector) and stage 3 ---------------------------------------------
   struct YPanel {
-    int64_t base = 0, rows = 0, K = 0, ld = 0;
+    int64_t base = 0, rows = 0, K = 0, ld = 0;    // reduced form: [rows x K]
+    int64_t kbase = 0, kld = 0;                   // FP64 form: [K x rows]
   };
   std::map<int, YPanel> ypn;
   // first Y row of (vec block vb, components c0, c1):
@@ -397,12 +438,13 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
   {
     std::map<int, std::vector<int64_t>> V_by_right;
     for (size_t vb = 0; vb < p.vec.blk.size(); ++vb) V_by_right[p.vec.blk[vb][bax]].push_back(vb);
-    int64_t ybase = 0;
+    int64_t ybase = 0, ykbase = 0;
     for (auto &kv : V_by_right) {
       const int bp = kv.first;
       auto pit = rpn.find(bp);
       YPanel Y;
       Y.base = ybase;
+      Y.kbase = ykbase;
       Y.K = pit == rpn.end() ? 0 : pit->second.K;
       Y.ld = ld8(Y.K);
       const int64_t Dbp = R.ax[0].deg[bp];
@@ -432,26 +474,37 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
       t.c_rowtab = 1;
       t.seg_begin = (int32_t)s3.segs.size();
       t.seg_count = 0;
+      Y.kld = ld16(Y.rows, Y.K);
       if (Y.K > 0) {
         GemmSeg g{};
         g.a_slot = SLOT_Y;
+        g.a_off = Y.kbase;
+        g.lda = Y.kld;
+        g.b_slot = SLOT_R;
+        g.b_off = pit->second.kbase;
+        g.ldb = pit->second.kld;
+        g.K = (int32_t)Y.K;
+        g.flags = SEG_TRANS_A;
+        s3.segs.push_back(g);
         g.a_off = Y.base;
         g.lda = Y.ld;
-        g.b_slot = SLOT_R;
         g.b_off = pit->second.base;
         g.ldb = pit->second.ld;
-        g.K = (int32_t)Y.K;
         g.flags = SEG_TRANS_B;
-        s3.segs.push_back(g);
+        r3.segs.push_back(g);
         t.seg_count = 1;
         s3.flops += fl * double(Y.rows) * double(Dbp) * double(Y.K);
       }
       s3.tasks.push_back(t);
+      r3.tasks.push_back(t);
       ybase += Y.rows * Y.ld;
+      ykbase += Y.K * Y.kld;
       y_alg += Y.rows * Y.K;
       ypn[bp] = Y;
     }
-    p.y_elems = ybase;
+    p.y_elems = ykbase;
+    p.yred_elems = ybase;
+    r3.crows = s3.crows;
   }
 
   pt.mark("stage3");
@@ -474,7 +527,7 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
   const auto so_z = sector_offsets(W1.ax[3]);
   using Key7 = std::array<int32_t, 7>;   // (t0 sect, t0 comp, t1 sect, t1 comp, z sect, z comp, b' sect)
   struct InRow {
-    RowDesc d;
+    RowDesc d, rd;   // FP64 form, reduced form
     int64_t wg, sg0, sg1;
     int wsec, ssec0, ssec1;
   };
@@ -493,7 +546,7 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
     for (auto &lr : stk.roff) {
       const int64_t lb = lr.first;
       const Coords &l = L.blk[lb];
-      const int64_t Wm = L.ax[1].deg[l[1]];
+      const int64_t Wm = L.ax[1].deg[l[1]], Dap = L.ax[0].deg[l[0]], tb = tbase[a];
       for (int64_t vb : V_by_left[a]) {
         const Coords &v = p.vec.blk[vb];
         const int b = v[bax];
@@ -513,8 +566,11 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
           for (int c0 = 0; c0 < d0; ++c0)
             for (int c1 = 0; c1 < d1; ++c1) {
               InRow r;
-              r.d.off = tbase[a] + (lr.second + w) * Na + fcol[vb] + (c0 * d1 + c1) * Db;
-              r.d.rs = Wm * Na;
+              const int64_t n0 = fcol[vb] + (c0 * d1 + c1) * Db;
+              r.d.off = tb + n0 * stk.rows + lr.second + w * Dap;
+              r.d.rs = stk.rows;
+              r.rd.off = tb + (lr.second + w) * Na + n0;
+              r.rd.rs = Wm * Na;
               r.wg = so_w0[l[1]] + w;
               r.sg0 = so_s[0][v[1]] + c0;
               r.sg1 = nphys == 2 ? so_s[1][v[2]] + c1 : 0;
@@ -561,7 +617,7 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
   // descriptors and its combined operator.  The lists are then joined in
   // channel order, so the plan is the same for any thread count.
   struct ChanBuilt {
-    std::vector<RowDesc> orows;
+    std::vector<RowDesc> orows, rorows;   // FP64 form, reduced form
     std::vector<double> coef;
   };
   std::vector<ChanBuilt> built(ch.size());
@@ -618,6 +674,7 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
     if (c.out.empty() || c.in.empty()) return;
     const int64_t Db = psi.ax[bax].deg[c.b];
     cb.orows.reserve(c.out.size());
+    cb.rorows.reserve(c.out.size());
     for (const Key7 &o : c.out) {
       const int bp = o[6];
       Coords ob{};
@@ -634,10 +691,9 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
       QLG_CHECK(yrow0[vb] >= 0 && cit != rit->second.col.end(), "planner: channel output lost");
       const YPanel &Y = yit->second;
       const int64_t row0 = yrow0[vb] + (int64_t)o[1] * ystep0[vb] + (int64_t)o[3] * ystep1[vb];
-      RowDesc d;
-      d.off = Y.base + row0 * Y.ld + cit->second + (int64_t)o[5] * Db;
-      d.rs = Y.ld;
-      cb.orows.push_back(d);
+      const int64_t k0 = cit->second + (int64_t)o[5] * Db;
+      cb.orows.push_back(RowDesc{Y.kbase + k0 * Y.kld + row0, Y.kld});
+      cb.rorows.push_back(RowDesc{Y.base + row0 * Y.ld + k0, Y.ld});
     }
     // combined operator rows (outputs) x columns (inputs)
     const int64_t K = (int64_t)c.in.size();
@@ -678,14 +734,20 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
     t.kin = (int32_t)c.in.size();
     t.kout = (int32_t)c.out.size();
     t.P = (int32_t)(Dap * Db);
-    t.Db = (int32_t)Db;
     t.in_rows = (int32_t)s2.rows.size();
-    for (const InRow &r : c.in) s2.rows.push_back(r.d);
+    for (const InRow &r : c.in) {
+      s2.rows.push_back(r.d);
+      r2.rows.push_back(r.rd);
+    }
     t.out_rows = (int32_t)s2.rows.size();
     s2.rows.insert(s2.rows.end(), built[ci].orows.begin(), built[ci].orows.end());
+    r2.rows.insert(r2.rows.end(), built[ci].rorows.begin(), built[ci].rorows.end());
     Ch.insert(Ch.end(), built[ci].coef.begin(), built[ci].coef.end());
     coff += (int64_t)c.out.size() * (int64_t)c.in.size();
+    t.Db = (int32_t)Dap;   // positions n = b * D_a' + a'
     s2.chan.push_back(t);
+    t.Db = (int32_t)Db;    // positions n = a' * D_b + b
+    r2.chan.push_back(t);
     s2.flops += fl * double(t.kout) * double(t.kin) * double(t.P);
   }
   p.c_elems = coff;
@@ -701,6 +763,12 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
     slot_elems[SLOT_Y] = p.y_elems;
     slot_elems[SLOT_C] = p.c_elems;
     for (int i = 0; i < 3; ++i) validate_stage(p.st[i], slot_elems);
+    slot_elems[SLOT_L] = lred_elems;
+    slot_elems[SLOT_R] = rred_elems;
+    slot_elems[SLOT_Y] = p.yred_elems;
+    for (int i = 0; i < 3; ++i) validate_stage(p.rst[i], slot_elems);
+    s1.find_direct();
+    s3.find_direct();
     // the MPO stage gathers from the whole first intermediate through 32-bit
     // byte offsets, and reads each channel operator the same way
     if (p.x_elems * ed * 8 >= (int64_t(1) << 31))
@@ -719,40 +787,24 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
     };
     check_copies(p.pack_in, p.vec.size, p.vec.size, "pack");
     check_copies(p.pack_out, p.vec.size, p.vec.size, "unpack");
-    check_copies(lcopy, extent(L), lint_elems, "L repack");
-    check_copies(rcopy, extent(R), rint_elems, "R repack");
+    auto check_trans = [](const std::vector<TransDesc> &v, int64_t src_n, int64_t dst_n, const char *what) {
+      for (const TransDesc &c : v)
+        QLG_CHECK(c.nz > 0 && c.nx > 0 && c.src >= 0 && c.dst >= 0 && c.sld >= c.nx && c.dsx >= c.nz &&
+                      c.src + (int64_t)(c.nz - 1) * c.sld + c.nx <= src_n &&
+                      c.dst + (int64_t)(c.nx - 1) * c.dsx + c.nz <= dst_n,
+                  std::string("copy list out of bounds: ") + what);
+    };
+    check_trans(lcopy, extent(L), lint_elems, "L repack");
+    check_trans(rcopy, extent(R), rint_elems, "R repack");
+    check_trans(p.red_l, lint_elems, lred_elems, "L reduced form");
+    check_trans(p.red_r, rint_elems, rred_elems, "R reduced form");
   }
-  const char *pin = std::getenv("QLG_TILES");
-  int pinned[3][2] = {{0, 0}, {0, 0}, {0, 0}};
-  if (pin) std::sscanf(pin, "%dx%d,%dx%d,%dx%d", &pinned[0][0], &pinned[0][1], &pinned[1][0], &pinned[1][1],
-                       &pinned[2][0], &pinned[2][1]);
   for (int i = 0; i < 3; ++i) {
-    if (pinned[i][0] > 0) {
-      p.st[i].make_tiles(pinned[i][0], pinned[i][1]);
-      p.tiles_pinned = true;
-    } else if (i == 1) {
-      // MPO stage: HBM-bound.  X is re-read once per row tile, so the row
-      // tile covers K_out where the MFMA padding stays cheap; the cost counts
-      // X reads per row tile plus padded MFMA work at ~10 flops per byte
-      double best = 1e300;
-      int bm_best = 32;
-      for (int bm : {16, 32, 64}) {
-        double cost = 0;
-        for (const ChanTask &c : s2.chan) {
-          const double rt = (c.kout + bm - 1) / bm;
-          cost += rt * c.kin * double(c.P) * 8.0 + rt * bm * double(c.kin) * c.P * 2.0 / 10.0;
-        }
-        if (cost < best) {
-          best = cost;
-          bm_best = bm;
-        }
-      }
-      p.st[i].make_tiles(bm_best, bm_best == 64 ? 64 : 128);
-    } else {
-      model_tiles(p.st[i], p.dtype == QLG_C128);   // replaced by measured shapes on the first matvec
-    }
-    p.st[i].upload(ctx->stream);
+    p.rst[i].flops = p.st[i].flops;
+    p.rst[i].algo_flops = p.st[i].algo_flops;
   }
+  if (const char *pin = std::getenv("QLG_TILES")) p.tile_pin = pin;
+  p.prepare_lists();
   pt.mark("tiles");
   p.d_pack_in.ensure(std::max<size_t>(1, p.pack_in.size()) * sizeof(CopyDesc));
   p.d_pack_out.ensure(std::max<size_t>(1, p.pack_out.size()) * sizeof(CopyDesc));
@@ -764,14 +816,15 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
   }
   const size_t eb = ed * sizeof(double);
   p.X.ensure(std::max<int64_t>(p.x_elems, 1) * eb);
-  p.Y.ensure(std::max<int64_t>(p.y_elems, 1) * eb);
+  p.Y.ensure((p.y_elems + 2) * eb);
   p.C.ensure(std::max<int64_t>(p.c_elems, 1) * eb);
-  p.Lint.ensure(std::max<int64_t>(lint_elems, 1) * eb);
-  p.Rint.ensure(std::max<int64_t>(rint_elems, 1) * eb);
+  p.Lint.ensure((lint_elems + 2) * eb);
+  p.Rint.ensure((rint_elems + 2) * eb);
   p.lint_elems = lint_elems;
   p.rint_elems = rint_elems;
-  // padding columns of the stacks and panels stay zero (the split-BF16
-  // kernels read them)
+  p.lred_elems = lred_elems;
+  p.rred_elems = rred_elems;
+  // the padding columns hold zeros
   QLG_HIP(hipMemsetAsync(p.Lint.p, 0, std::max<int64_t>(lint_elems, 1) * eb, ctx->stream));
   QLG_HIP(hipMemsetAsync(p.Rint.p, 0, std::max<int64_t>(rint_elems, 1) * eb, ctx->stream));
   pt.mark("alloc");
@@ -781,15 +834,15 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
     QLG_HIP(hipMemcpyAsync(p.C.p, Ch.data(), p.c_elems * eb, hipMemcpyHostToDevice, ctx->stream));
   {
     DevBuf dl, dr;
-    dl.ensure(std::max<size_t>(1, lcopy.size()) * sizeof(CopyDesc));
-    dr.ensure(std::max<size_t>(1, rcopy.size()) * sizeof(CopyDesc));
+    dl.ensure(std::max<size_t>(1, lcopy.size()) * sizeof(TransDesc));
+    dr.ensure(std::max<size_t>(1, rcopy.size()) * sizeof(TransDesc));
     if (!lcopy.empty())
-      QLG_HIP(hipMemcpyAsync(dl.p, lcopy.data(), lcopy.size() * sizeof(CopyDesc), hipMemcpyHostToDevice, ctx->stream));
+      QLG_HIP(hipMemcpyAsync(dl.p, lcopy.data(), lcopy.size() * sizeof(TransDesc), hipMemcpyHostToDevice, ctx->stream));
     if (!rcopy.empty())
-      QLG_HIP(hipMemcpyAsync(dr.p, rcopy.data(), rcopy.size() * sizeof(CopyDesc), hipMemcpyHostToDevice, ctx->stream));
-    launch_block_copy(ed == 2, dl.as<CopyDesc>(), (int)lcopy.size(), static_cast<const double *>(L.data),
+      QLG_HIP(hipMemcpyAsync(dr.p, rcopy.data(), rcopy.size() * sizeof(TransDesc), hipMemcpyHostToDevice, ctx->stream));
+    launch_tile_trans(ed == 2, dl.as<TransDesc>(), (int)lcopy.size(), static_cast<const double *>(L.data),
                       p.Lint.as<double>(), ctx->stream);
-    launch_block_copy(ed == 2, dr.as<CopyDesc>(), (int)rcopy.size(), static_cast<const double *>(R.data),
+    launch_tile_trans(ed == 2, dr.as<TransDesc>(), (int)rcopy.size(), static_cast<const double *>(R.data),
                       p.Rint.as<double>(), ctx->stream);
     QLG_HIP(hipStreamSynchronize(ctx->stream));
   }
@@ -800,17 +853,18 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
     p.st[0].algo_bytes = e8 * double(lint_alg + p.vec.size + p.x_elems);
     p.st[1].algo_bytes = e8 * double(p.x_elems + p.c_elems + y_alg);
     p.st[2].algo_bytes = e8 * double(y_alg + rint_alg + p.vec.size);
+    for (int i = 0; i < 3; ++i) p.rst[i].algo_bytes = p.st[i].algo_bytes;
   }
   if (const char *v = std::getenv("QLG_VERBOSE"); v && v[0] == '1') {
     const char *names[3] = {"L.psi", "MPO", ".R^T"};
     for (int i = 0; i < 3; ++i) {
-      const Stage &s = p.st[i];
+      const Stage &s = p.stage(i);
       std::fprintf(stderr, "[qlg plan] stage %d (%s): tasks %zu tiles %zu tile %dx%d gflop %.3f\n", i + 1, names[i],
                    i == 1 ? s.chan.size() : s.tasks.size(), s.tiles.size(), s.bm, s.bn, s.flops / 1e9);
     }
     for (int i : {0, 2}) {
       // tile efficiency (useful / padded MFMA work) and the task shape spread
-      const Stage &s = p.st[i];
+      const Stage &s = p.stage(i);
       double useful = 0, padded = 0;
       std::vector<int> ms, ns, ks;
       for (const GemmTask &k : s.tasks) {
@@ -843,12 +897,12 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
                  (long long)lint_elems, (long long)rint_elems, p.algo_flops / 1e9);
     int kin_max = 0, kout_max = 0, p_max = 0, nbig = 0;
     double xreads = 0, kin_avg = 0, kout_avg = 0, wsum = 0;
-    for (const ChanTask &c : s2.chan) {
+    for (const ChanTask &c : p.stage(1).chan) {
       kin_max = std::max(kin_max, c.kin);
       kout_max = std::max(kout_max, c.kout);
       p_max = std::max(p_max, c.P);
       nbig += c.kin > 256;
-      xreads += double((c.kout + s2.bm - 1) / s2.bm) * c.kin * c.P;
+      xreads += double((c.kout + p.stage(1).bm - 1) / p.stage(1).bm) * c.kin * c.P;
       kin_avg += double(c.kin) * c.P;
       kout_avg += double(c.kout) * c.P;
       wsum += c.P;
@@ -857,7 +911,7 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
                  "[qlg plan] MPO channels: kin max %d avg %.1f, kout max %d avg %.1f, P max %d avg %.0f, "
                  "kin>256: %d, X element reads %.0f (%.2fx T1)\n",
                  kin_max, kin_avg / std::max(wsum, 1.0), kout_max, kout_avg / std::max(wsum, 1.0), p_max,
-                 wsum / std::max<size_t>(s2.chan.size(), 1), nbig, xreads, xreads / std::max<double>(p.x_elems, 1));
+                 wsum / std::max<size_t>(p.stage(1).chan.size(), 1), nbig, xreads, xreads / std::max<double>(p.x_elems, 1));
   }
   return P.release();
 }
@@ -869,6 +923,50 @@ Plan::~Plan() {
   drop_graphs();
   if (host_seg) (void)hipHostFree(host_seg);
   if (host_lz) (void)hipHostFree(host_lz);
+}
+
+// Tile lists and uploads of the form the current precision uses, on its first
+// use.
+void Plan::prepare_lists() {
+  const int form = precision == QLG_PREC_F64 ? 0 : 1;
+  if (lists_ready[form]) return;
+  int pinned[3][2] = {{0, 0}, {0, 0}, {0, 0}};
+  if (!tile_pin.empty())
+    std::sscanf(tile_pin.c_str(), "%dx%d,%dx%d,%dx%d", &pinned[0][0], &pinned[0][1], &pinned[1][0], &pinned[1][1],
+                       &pinned[2][0], &pinned[2][1]);
+  for (int i = 0; i < 3; ++i) {
+    Stage &g = stage(i);
+    if (pinned[i][0] > 0) {
+      g.make_tiles(pinned[i][0], pinned[i][1]);
+      tiles_pinned = true;
+    } else if (i == 1) {
+      // MPO stage: HBM-bound.  X is re-read once per row tile, so the row
+      // tile covers K_out where the MFMA padding stays cheap; the cost counts
+      // X reads per row tile plus padded MFMA work at ~10 flops per byte
+      double best = 1e300;
+      int bm_best = 32;
+      for (int bm : {16, 32, 64}) {
+        double cost = 0;
+        for (const ChanTask &c : g.chan) {
+          const double rt = (c.kout + bm - 1) / bm;
+          cost += rt * c.kin * double(c.P) * 8.0 + rt * bm * double(c.kin) * c.P * 2.0 / 10.0;
+        }
+        if (cost < best) {
+          best = cost;
+          bm_best = bm;
+        }
+      }
+      g.make_tiles(bm_best, bm_best == 64 ? 64 : 128);
+    } else {
+      model_tiles(g, dtype == QLG_C128);   // replaced by measured shapes on the first matvec
+    }
+    g.upload(ctx->stream);
+  }
+  lists_ready[form] = true;
+}
+
+int64_t Plan::vec_bytes() const {
+  return (std::max<int64_t>(vec.size, 1) + 1) * elem_doubles(dtype) * (int64_t)sizeof(double);
 }
 
 void Plan::drop_graphs() {
@@ -894,33 +992,44 @@ bool Plan::planar() const {
 }
 
 void Plan::prepare_reduced() {
+  if (planar() ? planar_ready : reduced_ready) return;
+  // the reduced form's L stacks and R panels, from the FP64 form's
+  const int64_t ed = elem_doubles(dtype);   // complex data: (re, im) pairs of floats
+  DevBuf Lr, Rr, dl, dr;
+  for (auto &[buf, n, descs, dd, src] :
+       {std::tie(Lr, lred_elems, red_l, dl, Lint), std::tie(Rr, rred_elems, red_r, dr, Rint)}) {
+    const size_t bytes = (size_t)std::max<int64_t>(n, 1) * ed * sizeof(double);
+    buf.ensure(bytes);
+    QLG_HIP(hipMemsetAsync(buf.p, 0, bytes, ctx->stream));
+    if (descs.empty()) continue;
+    dd.ensure(descs.size() * sizeof(TransDesc));
+    QLG_HIP(hipMemcpyAsync(dd.p, descs.data(), descs.size() * sizeof(TransDesc), hipMemcpyHostToDevice, ctx->stream));
+    launch_tile_trans(ed == 2, dd.as<TransDesc>(), (int)descs.size(), src.as<double>(), buf.as<double>(), ctx->stream);
+  }
   if (planar()) {
     // real split-BF16: L stacks and R panels split once into three bf16 piece
     // planes; Y kept as planes written by the MPO stage (padding and entries
     // no channel writes stay zero); the channel operators in FP32
-    if (planar_ready) return;
-    Lp.ensure(std::max<int64_t>(3 * lint_elems, 1) * 2);
-    Rp.ensure(std::max<int64_t>(3 * rint_elems, 1) * 2);
-    Yp.ensure(std::max<int64_t>(3 * y_elems, 1) * 2);
+    Lp.ensure(std::max<int64_t>(3 * lred_elems, 1) * 2);
+    Rp.ensure(std::max<int64_t>(3 * rred_elems, 1) * 2);
+    Yp.ensure(std::max<int64_t>(3 * yred_elems, 1) * 2);
     C32.ensure(std::max<int64_t>(c_elems, 1) * sizeof(float));
-    QLG_HIP(hipMemsetAsync(Yp.p, 0, std::max<int64_t>(3 * y_elems, 1) * 2, ctx->stream));
-    launch_split_planes(Lint.as<double>(), Lp.p, lint_elems, ctx->stream);
-    launch_split_planes(Rint.as<double>(), Rp.p, rint_elems, ctx->stream);
+    QLG_HIP(hipMemsetAsync(Yp.p, 0, std::max<int64_t>(3 * yred_elems, 1) * 2, ctx->stream));
+    launch_split_planes(Lr.as<double>(), Lp.p, lred_elems, ctx->stream);
+    launch_split_planes(Rr.as<double>(), Rp.p, rred_elems, ctx->stream);
     launch_f64_to_f32(C.as<double>(), C32.as<float>(), c_elems, ctx->stream);
     planar_ready = true;
-    return;
+  } else {
+    Lint32.ensure(std::max<int64_t>(lred_elems * ed, 1) * sizeof(float));
+    Rint32.ensure(std::max<int64_t>(rred_elems * ed, 1) * sizeof(float));
+    C32.ensure(std::max<int64_t>(c_elems * ed, 1) * sizeof(float));
+    Y32.ensure(std::max<int64_t>(yred_elems * ed, 1) * sizeof(float));
+    QLG_HIP(hipMemsetAsync(Y32.p, 0, std::max<int64_t>(yred_elems * ed, 1) * sizeof(float), ctx->stream));
+    launch_f64_to_f32(Lr.as<double>(), Lint32.as<float>(), lred_elems * ed, ctx->stream);
+    launch_f64_to_f32(Rr.as<double>(), Rint32.as<float>(), rred_elems * ed, ctx->stream);
+    launch_f64_to_f32(C.as<double>(), C32.as<float>(), c_elems * ed, ctx->stream);
+    reduced_ready = true;
   }
-  if (reduced_ready) return;
-  const int64_t ed = elem_doubles(dtype);   // complex data: (re, im) pairs of floats
-  Lint32.ensure(std::max<int64_t>(lint_elems * ed, 1) * sizeof(float));
-  Rint32.ensure(std::max<int64_t>(rint_elems * ed, 1) * sizeof(float));
-  C32.ensure(std::max<int64_t>(c_elems * ed, 1) * sizeof(float));
-  Y32.ensure(std::max<int64_t>(y_elems * ed, 1) * sizeof(float));
-  QLG_HIP(hipMemsetAsync(Y32.p, 0, std::max<int64_t>(y_elems * ed, 1) * sizeof(float), ctx->stream));
-  launch_f64_to_f32(Lint.as<double>(), Lint32.as<float>(), lint_elems * ed, ctx->stream);
-  launch_f64_to_f32(Rint.as<double>(), Rint32.as<float>(), rint_elems * ed, ctx->stream);
-  launch_f64_to_f32(C.as<double>(), C32.as<float>(), c_elems * ed, ctx->stream);
-  reduced_ready = true;
 }
 
 Slots Plan::slots(const double *in, double *out) {
@@ -937,12 +1046,12 @@ Slots Plan::slots(const double *in, double *out) {
     s.p[SLOT_L] = static_cast<double *>(Lp.p);
     s.p[SLOT_R] = static_cast<double *>(Rp.p);
     s.p[SLOT_Y] = static_cast<double *>(Yp.p);
-    s.ps[SLOT_L] = lint_elems;
-    s.ps[SLOT_R] = rint_elems;
-    s.ps[SLOT_Y] = y_elems;
+    s.ps[SLOT_L] = lred_elems;
+    s.ps[SLOT_R] = rred_elems;
+    s.ps[SLOT_Y] = yred_elems;
   }
-  s.p[SLOT_W] = st[2].work.as<double>();
-  s.crows = st[2].d_crows.as<int64_t>();
+  s.p[SLOT_W] = stage(2).work.as<double>();
+  s.crows = stage(2).d_crows.as<int64_t>();
   s.skip = skip_flag;
   return s;
 }
@@ -950,10 +1059,10 @@ Slots Plan::slots(const double *in, double *out) {
 void Plan::launch_stage(int i, const Slots &s) {
   const bool reduced = precision != QLG_PREC_F64, cplx = dtype == QLG_C128;
   hipStream_t stream = ctx->stream;
-  Stage &g = st[i];
+  Stage &g = stage(i);
   const int out_planes = planar() ? (precision == QLG_PREC_BF16X6 ? 3 : 2) : 0;
   if (i == 1) {
-    launch_mpo_stage(g.bm, g.bn, cplx, reduced, out_planes, y_elems, g.d_ctiles.as<ChanTile>(),
+    launch_mpo_stage(g.bm, g.bn, cplx, reduced, out_planes, yred_elems, g.d_ctiles.as<ChanTile>(),
                      g.d_rows.as<RowDesc>(), s.p[SLOT_C], X.p, s.p[SLOT_Y], s.skip, (int)g.ctiles.size(), stream);
     return;
   }
@@ -968,6 +1077,9 @@ void Plan::launch_stage(int i, const Slots &s) {
     // stage 3: A = Y, B = R panels (transposed), C = the Krylov output (FP64, row table)
     launch_grouped_gemm_mixed(precision, g.bm, g.bn, i == 0, i == 2, cplx, g.d_tiles.as<GemmTile>(),
                               g.d_tasks.as<GemmTask>(), g.d_segs.as<GemmSeg>(), s, (int)g.tiles.size(), stream);
+  } else if (g.direct) {
+    launch_direct_gemm_f64(g.bm, g.bn, cplx, g.d_tiles.as<GemmTile>(), g.d_tasks.as<GemmTask>(),
+                           g.d_segs.as<GemmSeg>(), s, (int)g.tiles.size(), stream);
   } else {
     launch_grouped_gemm_f64(g.bm, g.bn, cplx, g.d_tiles.as<GemmTile>(), g.d_tasks.as<GemmTask>(),
                             g.d_segs.as<GemmSeg>(), s, (int)g.tiles.size(), stream);
@@ -1021,7 +1133,7 @@ void Plan::autotune(const double *in, double *out) {
   {
     std::lock_guard<std::mutex> lk(g_tile_mu);
     for (int i : {0, 2}) {
-      const Stage &g = st[i];
+      const Stage &g = stage(i);
       if (g.tasks.empty()) continue;
       auto it = g_tile_cache.find(tile_signature(g, i, variant));
       if (it != g_tile_cache.end()) {
@@ -1045,7 +1157,7 @@ void Plan::autotune(const double *in, double *out) {
   QLG_HIP(hipEventCreate(&e1));
   try {
     for (int i : {0, 2}) {
-      Stage &g = st[i];
+      Stage &g = stage(i);
       if (g.tasks.empty()) continue;
       TileChoice chosen = cached[i];
       if (chosen.bm == 0) {
@@ -1114,13 +1226,13 @@ void Plan::autotune(const double *in, double *out) {
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (verbose)
-    std::fprintf(stderr, "[qlg tune] tiles %dx%d / %dx%d%s (cache hits %d, misses %d)\n", st[0].bm, st[0].bn,
-                 st[2].bm, st[2].bn, st[2].split() ? " split-K" : "", g_tune_hits, g_tune_misses);
+    std::fprintf(stderr, "[qlg tune] tiles %dx%d / %dx%d%s (cache hits %d, misses %d)\n", stage(0).bm, stage(0).bn,
+                 stage(2).bm, stage(2).bn, stage(2).split() ? " split-K" : "", g_tune_hits, g_tune_misses);
   const char *vv = std::getenv("QLG_VERBOSE");
   if (vv && vv[0] == '3') {
     // task shapes of the two GEMM stages: FLOP-weighted quantiles of M, N, K
     for (int i : {0, 2}) {
-      const Stage &g = st[i];
+      const Stage &g = stage(i);
       std::vector<std::array<double, 4>> v;   // flops, M, N, K
       double tot = 0;
       for (const GemmTask &k : g.tasks) {
@@ -1154,6 +1266,7 @@ void Plan::autotune(const double *in, double *out) {
 void Plan::matvec_fused(const double *in, double *out) {
   const bool reduced = precision != QLG_PREC_F64;
   if (reduced) prepare_reduced();
+  prepare_lists();
   autotune(in, out);
   const Slots s = slots(in, out);
   hipStream_t stream = ctx->stream;
@@ -1170,9 +1283,8 @@ void Plan::matvec_fused(const double *in, double *out) {
 }
 
 void Plan::matvec(const double *in, double *out) {
-  const size_t bytes = std::max<int64_t>(vec.size, 1) * elem_doubles(dtype) * sizeof(double);
-  vtmp_in.ensure(bytes);
-  vtmp_out.ensure(bytes);
+  vtmp_in.ensure(vec_bytes());
+  vtmp_out.ensure(vec_bytes());
   to_fused(in, vtmp_in.as<double>());
   matvec_fused(vtmp_in.as<double>(), vtmp_out.as<double>());
   to_canonical(vtmp_out.as<double>(), out);

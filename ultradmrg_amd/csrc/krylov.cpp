@@ -54,7 +54,7 @@ struct Workspace {
     nslots = maxit + 1;
     if (p.basis_vectors < nslots) {
       p.basis.release();
-      p.basis.ensure((size_t)nslots * nd * sizeof(double));
+      p.basis.ensure((size_t)(nslots - 1) * nd * sizeof(double) + p.vec_bytes());
       p.basis_vectors = nslots;
     }
     slot0 = p.basis.as<double>();
@@ -75,7 +75,7 @@ struct Workspace {
   // y (canonical layout) <- sum_i coef_i * slot(i) for i < k (real or complex coefficients)
   void combine(int64_t k, const double *coefs, bool cplx_coef, double *y_canonical) {
     Ctx &c = *p.ctx;
-    p.vtmp_out.ensure((size_t)nd * sizeof(double));
+    p.vtmp_out.ensure(p.vec_bytes());
     double *y = p.vtmp_out.as<double>();
     std::vector<const double *> ptrs(k);
     for (int64_t i = 0; i < k; ++i) ptrs[i] = slot(i);
@@ -141,7 +141,7 @@ static void lanczos_gs_host(Plan &p, double *psi, const qlg_lanczos_params &prm,
       if (m == 1) {
         p.to_canonical(w.slot(0), psi);
         if (p.precision != QLG_PREC_F64) {
-          p.vtmp_out.ensure((size_t)w.nd * sizeof(double));
+          p.vtmp_out.ensure(p.vec_bytes());
           QLG_HIP(hipMemcpyAsync(p.vtmp_out.p, w.slot(0), (size_t)w.nd * sizeof(double), hipMemcpyDeviceToDevice,
                                  c.stream));
           energy0 = w.rayleigh_f64();
@@ -378,7 +378,7 @@ void lanczos_gs_batch(Plan &p, double *psi, const qlg_lanczos_params &prm, qlg_l
   std::vector<const double *> bp(k);
   for (int64_t j = 0; j < k; ++j) bp[j] = w.slot(j);
   QLG_HIP(hipMemcpyAsync(ptrs, bp.data(), sizeof(double *) * k, hipMemcpyHostToDevice, st));
-  p.vtmp_out.ensure((size_t)w.nd * sizeof(double));
+  p.vtmp_out.ensure(p.vec_bytes());
   seg_lincomb(st, tab, (int)k, coefs, ptrs, p.vtmp_out.as<double>());
   p.to_canonical(p.vtmp_out.as<double>(), psi);
   QLG_HIP(hipStreamSynchronize(st));
@@ -718,7 +718,7 @@ void lanczos_expmv(Plan &p, double *psi, double tau, const qlg_lanczos_params &p
   QLG_CHECK(cs.iters >= 1 && cs.iters <= maxit, "device expmv: invalid stop");
   iters = cs.iters;
   // psi <- ||psi_0|| sum_i c_i v_i with the device's coefficients
-  p.vtmp_out.ensure((size_t)w.nd * sizeof(double));
+  p.vtmp_out.ensure(p.vec_bytes());
   double *y = p.vtmp_out.as<double>();
   vec_lincomb(c, p.dtype, w.n, (int)iters, r.coef_cur, r.ptrs, true, 0.0, 0.0, false, y);
   vec_scal(c, p.dtype, w.n, initial_norm, 0.0, y);

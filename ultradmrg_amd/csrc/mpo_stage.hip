@@ -18,6 +18,8 @@
 // wait, so a chunk costs one memory latency.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "gemm.h"
 #include "tile_io.h"
@@ -300,6 +302,41 @@ __global__ __launch_bounds__(256) void trans_copy_kernel(const TransDesc *__rest
     else
       dst[c.dst + x * c.dsx + z] = src[c.src + z * c.sld + x];
   }
+}
+
+// the same copies for the environments' repack, in 32 x 32 tiles through LDS
+// so that both sides are touched in whole rows; blockIdx.y shares a
+// descriptor's tiles
+constexpr int kTransSplit = 16;
+template <bool CPLX>
+__global__ __launch_bounds__(256) void tile_trans_kernel(const TransDesc *__restrict__ d, const double *__restrict__ src,
+                                                         double *__restrict__ dst, int n) {
+  using E = typename std::conditional<CPLX, double2, double>::type;
+  __shared__ E t[32][33];
+  if ((int)blockIdx.x >= n) return;
+  const TransDesc c = d[blockIdx.x];
+  const E *S = reinterpret_cast<const E *>(src) + c.src;
+  E *D = reinterpret_cast<E *>(dst) + c.dst;
+  const int tz = (c.nz + 31) / 32, tx = (c.nx + 31) / 32;
+  const int lo = threadIdx.x & 31, hi = threadIdx.x >> 5;
+  for (int i = blockIdx.y; i < tz * tx; i += kTransSplit) {
+    const int z0 = i / tx * 32, x0 = i % tx * 32;
+    for (int r = hi; r < 32; r += 8)
+      if (z0 + r < c.nz && x0 + lo < c.nx) t[r][lo] = S[(int64_t)(z0 + r) * c.sld + x0 + lo];
+    __syncthreads();
+    for (int r = hi; r < 32; r += 8)
+      if (x0 + r < c.nx && z0 + lo < c.nz) D[(int64_t)(x0 + r) * c.dsx + z0 + lo] = t[lo][r];
+    __syncthreads();
+  }
+}
+
+void launch_tile_trans(bool cplx, const TransDesc *d, int n, const double *src, double *dst, hipStream_t st) {
+  if (n <= 0) return;
+  if (cplx)
+    hipLaunchKernelGGL(tile_trans_kernel<true>, dim3(n, kTransSplit), dim3(256), 0, st, d, src, dst, n);
+  else
+    hipLaunchKernelGGL(tile_trans_kernel<false>, dim3(n, kTransSplit), dim3(256), 0, st, d, src, dst, n);
+  QLG_HIP(hipGetLastError());
 }
 
 // the same copies with a source buffer per descriptor (many operators, one launch)

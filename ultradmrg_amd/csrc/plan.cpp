@@ -282,6 +282,25 @@ void make_tiles_lpt(std::vector<GemmTile> &tiles, const std::vector<std::array<i
   while (!tiles.empty() && tiles.back().task < 0) tiles.pop_back();
 }
 
+// The direct FP64 GEMM (gemm_f64.hip) takes A stored [K x M] and B stored
+// [K x N], unconjugated.  Real data is read in pairs that may reach one element
+// past an operand's last row, so its operands must be the plan's own (padded
+// panels, vectors with slack).  A slice's scalar offset reaches up to 15 rows
+// past K and has to stay below 2^31 bytes.  Other stages (the contractions
+// around the solve) run on the LDS kernel.
+void Stage::find_direct() {
+  direct = false;
+  for (const GemmTask &t : tasks)
+    for (int q = 0; q < t.seg_count; ++q) {
+      const GemmSeg &g = segs[t.seg_begin + q];
+      if (g.K <= 0) continue;
+      if (g.flags != SEG_TRANS_A) return;
+      if ((int64_t)(g.K + 16) * std::max(g.lda, g.ldb) * ed * 8 >= (int64_t(1) << 31)) return;
+      if ((g.a_slot != SLOT_IN && g.a_slot != SLOT_Y) || (g.b_slot != SLOT_L && g.b_slot != SLOT_R)) return;
+    }
+  direct = !tasks.empty();
+}
+
 void Stage::upload(hipStream_t st) {
   if (!chan.empty()) {
     d_chan.ensure(chan.size() * sizeof(ChanTask));

@@ -8,6 +8,7 @@
 // Tensordot and environment-update plans (ctr.cpp) reuse the grouped GEMM.
 #pragma once
 #include <memory>
+#include <string>
 #include <vector>
 
 #include "common.h"
@@ -36,6 +37,8 @@ struct Stage {
   bool splitk = false;             // the stage may run split-K parts
   bool split_on = false;           // make_tiles splits (the tuner's choice, or QLG_SPLITK)
   int ed = 1;                      // doubles per element (complex: 2)
+  bool direct = false;             // every task can run on the direct FP64 GEMM (set by find_direct)
+  void find_direct();
   int64_t kchunk = 0;              // 0: no task is split
   std::vector<GemmTask> ktasks;
   std::vector<GemmSeg> ksegs;
@@ -73,9 +76,21 @@ struct Plan {
   int precision = QLG_PREC_F64;
   Ten L, W[2], R;
   Layout vec;
-  Stage st[3];
+  // The FP64 form (st) keeps every operand of the two contractions with k as
+  // its row index: L stacks [D_a x rows], T1 [N_a x rows], Y [K x rows], R
+  // panels [K x D_b'] (what gemm_f64.hip reads in whole cache lines, and, with
+  // a' the contiguous index, what the MPO stage reads and writes in runs of
+  // D_a').  The reduced modes (rst) keep the transposed layouts, whose
+  // k-contiguous rows their 16-byte fragments need.  Tile lists and uploads of
+  // either form are made when it is first used.
+  Stage st[3], rst[3];
+  bool lists_ready[2] = {false, false};
+  Stage &stage(int i) { return precision == QLG_PREC_F64 ? st[i] : rst[i]; }
+  std::string tile_pin;         // QLG_TILES when the plan was built
+  void prepare_lists();
   DevBuf X, Y, C;
   int64_t x_elems = 0, y_elems = 0, c_elems = 0;
+  int64_t vec_bytes() const;    // a vector's buffer, with one element of slack
   double algo_flops = 0;
   // Krylov workspace
   DevBuf basis, coef_buf, ptr_buf, scal_buf;
@@ -95,12 +110,16 @@ struct Plan {
   // between it and the canonical layout of the boundary.
   std::vector<CopyDesc> pack_in, pack_out;
   DevBuf d_pack_in, d_pack_out;
-  DevBuf Lint, Rint;            // environments repacked (ket-major L stacks, bra-major R panels)
+  DevBuf Lint, Rint;            // environments repacked for the FP64 form
   int64_t lint_elems = 0, rint_elems = 0;
-  // reduced-precision modes: FP32 copies of the L stacks, R panels and
-  // channel operators (made on first use).  T1 reuses X (stage 1 rewrites
-  // all of it every matvec); Y32 is a buffer of its own because stage 3
-  // reads Y entries that no channel writes, which must stay zero.
+  // reduced-precision modes: their layouts' sizes, the copies that make their
+  // L stacks and R panels from Lint and Rint, and FP32 copies of the L stacks,
+  // R panels and channel operators (made on first use).
+  int64_t lred_elems = 0, rred_elems = 0, yred_elems = 0;
+  std::vector<TransDesc> red_l, red_r;
+  // T1 reuses X (stage 1 rewrites all of it every matvec); Y32 is a buffer of
+  // its own because stage 3 reads Y entries that no channel writes, which must
+  // stay zero.
   DevBuf Lint32, Rint32, C32, Y32;
   bool reduced_ready = false;
   // real split-BF16 modes: L stacks, R panels and Y as three bf16 piece
@@ -170,6 +189,7 @@ void launch_split_planes(const double *src, void *dst, int64_t n, hipStream_t st
 void launch_grouped_gemm_mixed(int mode, int bm, int bn, bool b_f64, bool c_f64, bool cplx, const GemmTile *tiles,
                                const GemmTask *tasks, const GemmSeg *segs, const Slots &slots, int ntiles,
                                hipStream_t st);
+void launch_tile_trans(bool cplx, const TransDesc *d, int n, const double *src, double *dst, hipStream_t st);
 void launch_f64_to_f32(const double *src, float *dst, int64_t n, hipStream_t st);
 void launch_block_copy(bool cplx, const CopyDesc *d, int n, const double *src, double *dst, hipStream_t st);
 void validate_stage(const Stage &s, const int64_t *slot_elems);
@@ -180,6 +200,9 @@ std::string tile_signature(const Stage &s, int stage, int variant);
 
 void launch_grouped_gemm_f64(int bm, int bn, bool cplx, const GemmTile *tiles, const GemmTask *tasks,
                              const GemmSeg *segs, const Slots &slots, int ntiles, hipStream_t st);
+// fragments straight from memory (gemm_f64.hip): a stage with Stage::direct set
+void launch_direct_gemm_f64(int bm, int bn, bool cplx, const GemmTile *tiles, const GemmTask *tasks,
+                            const GemmSeg *segs, const Slots &slots, int ntiles, hipStream_t st);
 // sums the split-K partial panels of a stage into its outputs (FP64 / complex128)
 void launch_splitk_reduce(bool cplx, const RedTask *red, const RedChunk *chunks, int nchunks, const Slots &slots,
                           hipStream_t st);
