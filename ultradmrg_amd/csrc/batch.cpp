@@ -104,6 +104,7 @@ Plan *build_batch_plan(Ctx *ctx, int64_t n, Plan *const *members) {
       }
       // row-table entries address the task's output slot (the Krylov output)
       for (int64_t r : s.crows) d.crows.push_back(r + b[SLOT_OUT]);
+      for (int64_t r : s.canon) d.canon.push_back(r + b[SLOT_OUT]);
       for (ChanTask c : s.chan) {
         for (int r = 0; r < c.kin; ++r) {
           RowDesc e = s.rows[c.in_rows + r];

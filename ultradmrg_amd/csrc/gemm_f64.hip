@@ -465,6 +465,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK, FM * FN * (CPLX ? 2 : 1) <= 8 ? 
       if (n + d + kDepth < ns) multiply(d);
   }
 
+  // output row addresses: a row-address table or a plain row stride
+  int64_t crow[FM][4];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = m0 + frag_pos<FM, CPLX>(i, (lane >> 4) + 4 * r);
+      crow[i][r] = tk.c_rowtab ? slots.crows[tk.c_row + min(row, M - 1)] : tk.c_off + (int64_t)row * tk.ldc;
+    }
+
   if constexpr (WK > 1) {   // sum the k parts, in order
     constexpr int R = NP * FM * FN * 4;
     __shared__ double red[(WK - 1) * WM * WN][R][64];
@@ -482,15 +492,6 @@ __global__ __launch_bounds__(64 * WM * WN * WK, FM * FN * (CPLX ? 2 : 1) <= 8 ? 
         acc[r / (FM * FN * 4)][r / (FN * 4) % FM][r / 4 % FN][r % 4] += red[q * WM * WN + wmn][r][lane];
   }
 
-  // output row addresses: a row-address table or a plain row stride
-  int64_t crow[FM][4];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = m0 + frag_pos<FM, CPLX>(i, (lane >> 4) + 4 * r);
-      crow[i][r] = tk.c_rowtab ? slots.crows[tk.c_row + min(row, M - 1)] : tk.c_off + (int64_t)row * tk.ldc;
-    }
   double *C = slots.p[tk.c_slot];
 #pragma unroll
   for (int i = 0; i < FM; ++i)

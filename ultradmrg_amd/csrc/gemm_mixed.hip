@@ -1020,30 +1020,6 @@ __global__ __launch_bounds__(256) void gemm_bf16p_kernel(const GemmTile *__restr
   store_tile<FM, FN, TC>(tk, tl, slots, wm0, wn0, lane, acc);
 }
 
-// FP64 -> NPIECE bf16 planes of the FP32 value (h, m, l), element for element:
-// the pre-split constant operands, made once per plan
-template <int NPIECE>
-__global__ __launch_bounds__(256) void split_planes_kernel(const double *__restrict__ src, __bf16 *__restrict__ dst,
-                                                           int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    float r = (float)src[i];
-#pragma unroll
-    for (int q = 0; q < NPIECE; ++q) {
-      const __bf16 h = (__bf16)r;
-      dst[q * n + i] = h;
-      r -= (float)h;
-    }
-  }
-}
-
-void launch_split_planes(const double *src, void *dst, int64_t n, hipStream_t st) {
-  if (n <= 0) return;
-  const int64_t blocks = std::min<int64_t>((n + 255) / 256, 65536);
-  hipLaunchKernelGGL(split_planes_kernel<3>, dim3((unsigned)blocks), dim3(256), 0, st, src,
-                     static_cast<__bf16 *>(dst), n);
-  QLG_HIP(hipGetLastError());
-}
-
 // stage 1 (A planar, B = the FP64 vector split at staging, FP32 out) or
 // stage 3 (A and B planar, FP64 out through the row table)
 void launch_grouped_gemm_planar(int mode, int bm, int bn, bool stage3, const GemmTile *tiles, const GemmTask *tasks,

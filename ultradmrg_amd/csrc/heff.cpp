@@ -24,7 +24,6 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <tuple>
 #include <unordered_map>
 #include <set>
 
@@ -460,7 +459,11 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
         for (int c0 = 0; c0 < d0; ++c0)
           for (int c1 = 0; c1 < d1; ++c1) {
             const int64_t col0 = fz[ap].base + fcol[vb] + (c0 * d1 + c1) * Dbp;
-            for (int64_t r = 0; r < Dap; ++r) s3.crows.push_back(col0 + r * fz[ap].N);
+            const int64_t can0 = p.vec.off[vb] + (c0 * d1 + c1) * Dbp;
+            for (int64_t r = 0; r < Dap; ++r) {
+              s3.crows.push_back(col0 + r * fz[ap].N);
+              s3.canon.push_back(can0 + r * d0 * d1 * Dbp);
+            }
             Y.rows += Dap;
           }
       }
@@ -505,6 +508,7 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
     p.y_elems = ykbase;
     p.yred_elems = ybase;
     r3.crows = s3.crows;
+    for (int64_t o : s3.canon) QLG_CHECK(o >= 0 && o < p.vec.size, "canonical row table out of range");
   }
 
   pt.mark("stage3");
@@ -785,6 +789,8 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
       for (size_t b = 0; b < t.blk.size(); ++b) e = std::max(e, t.off[b] + t.blk_elems(b));
       return e;
     };
+    split_copies(p.pack_in);
+    split_copies(p.pack_out);
     check_copies(p.pack_in, p.vec.size, p.vec.size, "pack");
     check_copies(p.pack_out, p.vec.size, p.vec.size, "unpack");
     auto check_trans = [](const std::vector<TransDesc> &v, int64_t src_n, int64_t dst_n, const char *what) {
@@ -840,10 +846,10 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
       QLG_HIP(hipMemcpyAsync(dl.p, lcopy.data(), lcopy.size() * sizeof(TransDesc), hipMemcpyHostToDevice, ctx->stream));
     if (!rcopy.empty())
       QLG_HIP(hipMemcpyAsync(dr.p, rcopy.data(), rcopy.size() * sizeof(TransDesc), hipMemcpyHostToDevice, ctx->stream));
-    launch_tile_trans(ed == 2, dl.as<TransDesc>(), (int)lcopy.size(), static_cast<const double *>(L.data),
-                      p.Lint.as<double>(), ctx->stream);
-    launch_tile_trans(ed == 2, dr.as<TransDesc>(), (int)rcopy.size(), static_cast<const double *>(R.data),
-                      p.Rint.as<double>(), ctx->stream);
+    launch_tile_trans(ed == 2, 0, dl.as<TransDesc>(), (int)lcopy.size(), static_cast<const double *>(L.data), p.Lint.p, 0,
+                      ctx->stream);
+    launch_tile_trans(ed == 2, 0, dr.as<TransDesc>(), (int)rcopy.size(), static_cast<const double *>(R.data), p.Rint.p, 0,
+                      ctx->stream);
     QLG_HIP(hipStreamSynchronize(ctx->stream));
   }
   pt.mark("repack+sync");
@@ -979,6 +985,19 @@ void Plan::drop_graphs() {
   chunk_key.clear();
 }
 
+// pieces of at most about 4096 elements, for block_copy_kernel
+void split_copies(std::vector<CopyDesc> &v) {
+  constexpr int64_t kCopyPiece = 4096;
+  std::vector<CopyDesc> out;
+  out.reserve(v.size());
+  for (const CopyDesc &c : v) {
+    const int32_t step = (int32_t)std::max<int64_t>(1, kCopyPiece / std::max(c.cols, 1));
+    for (int32_t r = 0; r < c.rows; r += step)
+      out.push_back(CopyDesc{c.src + r * c.sld, c.dst + r * c.dld, c.sld, c.dld, std::min(step, c.rows - r), c.cols});
+  }
+  v.swap(out);
+}
+
 void Plan::to_fused(const double *canon, double *fused) {
   launch_block_copy(dtype == QLG_C128, d_pack_in.as<CopyDesc>(), (int)pack_in.size(), canon, fused, ctx->stream);
 }
@@ -993,43 +1012,32 @@ bool Plan::planar() const {
 
 void Plan::prepare_reduced() {
   if (planar() ? planar_ready : reduced_ready) return;
-  // the reduced form's L stacks and R panels, from the FP64 form's
+  // L stacks and R panels made from the FP64 form's, transposed: three bf16
+  // piece planes each (real split-BF16, where the MPO stage writes Y as planes
+  // too), or FP32.  Padding, and Y entries that no channel writes, stay zero.
   const int64_t ed = elem_doubles(dtype);   // complex data: (re, im) pairs of floats
-  DevBuf Lr, Rr, dl, dr;
-  for (auto &[buf, n, descs, dd, src] :
-       {std::tie(Lr, lred_elems, red_l, dl, Lint), std::tie(Rr, rred_elems, red_r, dr, Rint)}) {
-    const size_t bytes = (size_t)std::max<int64_t>(n, 1) * ed * sizeof(double);
-    buf.ensure(bytes);
-    QLG_HIP(hipMemsetAsync(buf.p, 0, bytes, ctx->stream));
-    if (descs.empty()) continue;
+  const bool pl = planar();
+  const int64_t eb = pl ? 3 * 2 : ed * (int64_t)sizeof(float);   // bytes per element
+  DevBuf &Lo = pl ? Lp : Lint32, &Ro = pl ? Rp : Rint32, &Yo = pl ? Yp : Y32;
+  DevBuf dl, dr;
+  auto zeroed = [&](DevBuf &buf, int64_t n) {
+    buf.ensure((size_t)(std::max<int64_t>(n, 1) * eb));
+    QLG_HIP(hipMemsetAsync(buf.p, 0, (size_t)(std::max<int64_t>(n, 1) * eb), ctx->stream));
+  };
+  auto transposed = [&](const std::vector<TransDesc> &descs, DevBuf &dd, const DevBuf &src, DevBuf &out, int64_t n) {
+    zeroed(out, n);
+    if (descs.empty()) return;
     dd.ensure(descs.size() * sizeof(TransDesc));
     QLG_HIP(hipMemcpyAsync(dd.p, descs.data(), descs.size() * sizeof(TransDesc), hipMemcpyHostToDevice, ctx->stream));
-    launch_tile_trans(ed == 2, dd.as<TransDesc>(), (int)descs.size(), src.as<double>(), buf.as<double>(), ctx->stream);
-  }
-  if (planar()) {
-    // real split-BF16: L stacks and R panels split once into three bf16 piece
-    // planes; Y kept as planes written by the MPO stage (padding and entries
-    // no channel writes stay zero); the channel operators in FP32
-    Lp.ensure(std::max<int64_t>(3 * lred_elems, 1) * 2);
-    Rp.ensure(std::max<int64_t>(3 * rred_elems, 1) * 2);
-    Yp.ensure(std::max<int64_t>(3 * yred_elems, 1) * 2);
-    C32.ensure(std::max<int64_t>(c_elems, 1) * sizeof(float));
-    QLG_HIP(hipMemsetAsync(Yp.p, 0, std::max<int64_t>(3 * yred_elems, 1) * 2, ctx->stream));
-    launch_split_planes(Lr.as<double>(), Lp.p, lred_elems, ctx->stream);
-    launch_split_planes(Rr.as<double>(), Rp.p, rred_elems, ctx->stream);
-    launch_f64_to_f32(C.as<double>(), C32.as<float>(), c_elems, ctx->stream);
-    planar_ready = true;
-  } else {
-    Lint32.ensure(std::max<int64_t>(lred_elems * ed, 1) * sizeof(float));
-    Rint32.ensure(std::max<int64_t>(rred_elems * ed, 1) * sizeof(float));
-    C32.ensure(std::max<int64_t>(c_elems * ed, 1) * sizeof(float));
-    Y32.ensure(std::max<int64_t>(yred_elems * ed, 1) * sizeof(float));
-    QLG_HIP(hipMemsetAsync(Y32.p, 0, std::max<int64_t>(yred_elems * ed, 1) * sizeof(float), ctx->stream));
-    launch_f64_to_f32(Lr.as<double>(), Lint32.as<float>(), lred_elems * ed, ctx->stream);
-    launch_f64_to_f32(Rr.as<double>(), Rint32.as<float>(), rred_elems * ed, ctx->stream);
-    launch_f64_to_f32(C.as<double>(), C32.as<float>(), c_elems * ed, ctx->stream);
-    reduced_ready = true;
-  }
+    launch_tile_trans(ed == 2, pl ? 2 : 1, dd.as<TransDesc>(), (int)descs.size(), src.as<double>(), out.p, n,
+                      ctx->stream);
+  };
+  transposed(red_l, dl, Lint, Lo, lred_elems);
+  transposed(red_r, dr, Rint, Ro, rred_elems);
+  zeroed(Yo, yred_elems);
+  C32.ensure(std::max<int64_t>(c_elems * ed, 1) * sizeof(float));
+  launch_f64_to_f32(C.as<double>(), C32.as<float>(), c_elems * ed, ctx->stream);
+  (pl ? planar_ready : reduced_ready) = true;
 }
 
 Slots Plan::slots(const double *in, double *out) {
@@ -1263,12 +1271,13 @@ void Plan::autotune(const double *in, double *out) {
   }
 }
 
-void Plan::matvec_fused(const double *in, double *out) {
+void Plan::matvec_fused(const double *in, double *out, const int64_t *crows) {
   const bool reduced = precision != QLG_PREC_F64;
   if (reduced) prepare_reduced();
   prepare_lists();
   autotune(in, out);
-  const Slots s = slots(in, out);
+  Slots s = slots(in, out);
+  if (crows) s.crows = crows;
   hipStream_t stream = ctx->stream;
   const bool timed = timing && !capturing;
   if (timed) {
@@ -1284,10 +1293,15 @@ void Plan::matvec_fused(const double *in, double *out) {
 
 void Plan::matvec(const double *in, double *out) {
   vtmp_in.ensure(vec_bytes());
-  vtmp_out.ensure(vec_bytes());
+  const std::vector<int64_t> &canon = st[2].canon;
+  if (!d_canon.p && !canon.empty()) {
+    d_canon.ensure(canon.size() * sizeof(int64_t));
+    QLG_HIP(hipMemcpyAsync(d_canon.p, canon.data(), canon.size() * sizeof(int64_t), hipMemcpyHostToDevice,
+                           ctx->stream));
+  }
   to_fused(in, vtmp_in.as<double>());
-  matvec_fused(vtmp_in.as<double>(), vtmp_out.as<double>());
-  to_canonical(vtmp_out.as<double>(), out);
+  // stage 3 writes its rows where the canonical layout has them
+  matvec_fused(vtmp_in.as<double>(), out, d_canon.as<int64_t>());
 }
 
 }  // namespace qlg

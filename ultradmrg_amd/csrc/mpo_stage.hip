@@ -262,28 +262,25 @@ __global__ __launch_bounds__(256) void mpo_stage_kernel(const ChanTile *__restri
   }
 }
 
-// 2-D block copies: dst[r * dld + c] = src[r * sld + c] for each descriptor.
-// Workgroup (x, y) copies rows y, y + kCopySplit, ... of descriptor x; each
-// wave takes one row at a time and its lanes walk the columns, so loads and
-// stores are contiguous runs and no per-element division is needed.
-constexpr int kCopySplit = 8;
-
+// 2-D block copies: dst[r * dld + c] = src[r * sld + c] for each descriptor,
+// one workgroup each.  A power of two of threads walks a row, so that no
+// element needs a division; the lists are cut into pieces of about kCopyPiece
+// elements (split_copies), so that no workgroup has much more than the others:
+// with whole blocks and eight workgroups each, a converged state's largest
+// blocks took 33 us of a 23 MB copy, the pieces 9 us.
 template <bool CPLX>
 __global__ __launch_bounds__(256) void block_copy_kernel(const CopyDesc *__restrict__ d, const double *__restrict__ src,
                                                          double *__restrict__ dst, int n) {
-  const int i = blockIdx.x;
-  if (i >= n) return;
-  const CopyDesc c = d[i];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int r = blockIdx.y + kCopySplit * wave; r < c.rows; r += kCopySplit * 4) {
-    const int64_t so = c.src + (int64_t)r * c.sld, dof = c.dst + (int64_t)r * c.dld;
-    for (int col = lane; col < c.cols; col += 64) {
-      if constexpr (CPLX)
-        reinterpret_cast<double2 *>(dst)[dof + col] = reinterpret_cast<const double2 *>(src)[so + col];
-      else
-        dst[dof + col] = src[so + col];
-    }
-  }
+  using E = typename std::conditional<CPLX, double2, double>::type;
+  if ((int)blockIdx.x >= n) return;
+  const CopyDesc c = d[blockIdx.x];
+  const int lg = c.cols > 128 ? 8 : 32 - __clz(c.cols - 1);   // 2^lg >= cols, at most 256 threads a row
+  const int lo = threadIdx.x & ((1 << lg) - 1), hi = threadIdx.x >> lg;
+  const E *S = reinterpret_cast<const E *>(src) + c.src;
+  E *D = reinterpret_cast<E *>(dst) + c.dst;
+  for (int col = lo; col < c.cols; col += 256)
+#pragma unroll 4
+    for (int r = hi; r < c.rows; r += 256 >> lg) D[(int64_t)r * c.dld + col] = S[(int64_t)r * c.sld + col];
 }
 
 // transposed copies (stacking block operators): one workgroup per descriptor
@@ -306,17 +303,17 @@ __global__ __launch_bounds__(256) void trans_copy_kernel(const TransDesc *__rest
 
 // the same copies for the environments' repack, in 32 x 32 tiles through LDS
 // so that both sides are touched in whole rows; blockIdx.y shares a
-// descriptor's tiles
+// descriptor's tiles.  OUT: 0 FP64, 1 FP32, 2 three bf16 piece planes of the
+// FP32 value, ps elements apart (what the reduced modes read).
 constexpr int kTransSplit = 16;
-template <bool CPLX>
+template <bool CPLX, int OUT>
 __global__ __launch_bounds__(256) void tile_trans_kernel(const TransDesc *__restrict__ d, const double *__restrict__ src,
-                                                         double *__restrict__ dst, int n) {
+                                                         void *__restrict__ dst, int64_t ps, int n) {
   using E = typename std::conditional<CPLX, double2, double>::type;
   __shared__ E t[32][33];
   if ((int)blockIdx.x >= n) return;
   const TransDesc c = d[blockIdx.x];
   const E *S = reinterpret_cast<const E *>(src) + c.src;
-  E *D = reinterpret_cast<E *>(dst) + c.dst;
   const int tz = (c.nz + 31) / 32, tx = (c.nx + 31) / 32;
   const int lo = threadIdx.x & 31, hi = threadIdx.x >> 5;
   for (int i = blockIdx.y; i < tz * tx; i += kTransSplit) {
@@ -325,17 +322,42 @@ __global__ __launch_bounds__(256) void tile_trans_kernel(const TransDesc *__rest
       if (z0 + r < c.nz && x0 + lo < c.nx) t[r][lo] = S[(int64_t)(z0 + r) * c.sld + x0 + lo];
     __syncthreads();
     for (int r = hi; r < 32; r += 8)
-      if (x0 + r < c.nx && z0 + lo < c.nz) D[(int64_t)(x0 + r) * c.dsx + z0 + lo] = t[lo][r];
+      if (x0 + r < c.nx && z0 + lo < c.nz) {
+        const E v = t[lo][r];
+        const int64_t o = c.dst + (int64_t)(x0 + r) * c.dsx + z0 + lo;
+        if constexpr (OUT == 0) {
+          static_cast<E *>(dst)[o] = v;
+        } else if constexpr (OUT == 1) {
+          if constexpr (CPLX)
+            static_cast<float2 *>(dst)[o] = float2{(float)v.x, (float)v.y};
+          else
+            static_cast<float *>(dst)[o] = (float)v;
+        } else if constexpr (!CPLX) {
+          float x = (float)v;
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            const __bf16 h = (__bf16)x;
+            static_cast<__bf16 *>(dst)[q * ps + o] = h;
+            x -= (float)h;
+          }
+        }
+      }
     __syncthreads();
   }
 }
 
-void launch_tile_trans(bool cplx, const TransDesc *d, int n, const double *src, double *dst, hipStream_t st) {
+void launch_tile_trans(bool cplx, int out, const TransDesc *d, int n, const double *src, void *dst, int64_t ps,
+                       hipStream_t st) {
   if (n <= 0) return;
-  if (cplx)
-    hipLaunchKernelGGL(tile_trans_kernel<true>, dim3(n, kTransSplit), dim3(256), 0, st, d, src, dst, n);
-  else
-    hipLaunchKernelGGL(tile_trans_kernel<false>, dim3(n, kTransSplit), dim3(256), 0, st, d, src, dst, n);
+  const dim3 grid(n, kTransSplit), block(256);
+#define QLG_TRANS(C_, O_)                                                                                     \
+  if (cplx == C_ && out == O_) hipLaunchKernelGGL((tile_trans_kernel<C_, O_>), grid, block, 0, st, d, src, dst, ps, n);
+  QLG_TRANS(false, 0)
+  QLG_TRANS(true, 0)
+  QLG_TRANS(false, 1)
+  QLG_TRANS(true, 1)
+  QLG_TRANS(false, 2)
+#undef QLG_TRANS
   QLG_HIP(hipGetLastError());
 }
 
@@ -425,9 +447,9 @@ void launch_mpo_stage(int bm, int bn, bool cplx, bool f32, int out_planes, int64
 void launch_block_copy(bool cplx, const CopyDesc *d, int n, const double *src, double *dst, hipStream_t st) {
   if (n <= 0) return;
   if (cplx)
-    hipLaunchKernelGGL(block_copy_kernel<true>, dim3(n, kCopySplit), dim3(256), 0, st, d, src, dst, n);
+    hipLaunchKernelGGL(block_copy_kernel<true>, dim3(n), dim3(256), 0, st, d, src, dst, n);
   else
-    hipLaunchKernelGGL(block_copy_kernel<false>, dim3(n, kCopySplit), dim3(256), 0, st, d, src, dst, n);
+    hipLaunchKernelGGL(block_copy_kernel<false>, dim3(n), dim3(256), 0, st, d, src, dst, n);
   QLG_HIP(hipGetLastError());
 }
 

@@ -21,6 +21,7 @@ struct Stage {
   std::vector<GemmTask> tasks;
   std::vector<GemmSeg> segs;
   std::vector<int64_t> crows;      // output-row address table (tasks with c_rowtab)
+  std::vector<int64_t> canon;      // the same rows in the canonical layout (stage 3 of qlg_matvec)
   std::vector<ChanTask> chan;      // MPO-stage channels (instead of tasks)
   std::vector<RowDesc> rows;       // their gathered / scattered rows
   std::vector<ChanTile> ctiles;    // MPO stage: tiles with their channels inlined (upload)
@@ -128,6 +129,7 @@ struct Plan {
   bool planar_ready = false;
   bool planar() const;
   void prepare_reduced();
+  DevBuf d_canon;               // row table of the canonical output (made on the first qlg_matvec)
   DevBuf vtmp_in, vtmp_out;     // staging for qlg_matvec on canonical vectors
   // batch plans: member m's vector occupies [batch_off[m], batch_off[m+1])
   // of the batch vector (canonical and fused layouts alike)
@@ -157,7 +159,8 @@ struct Plan {
   int64_t perm_n = 0, perm_maxel = 0;
   ~Plan();
   void matvec(const double *in, double *out);        // canonical in / out
-  void matvec_fused(const double *in, double *out);  // fused in / out
+  // fused in, fused out (or, with `crows`, rows of the output where that table puts them)
+  void matvec_fused(const double *in, double *out, const int64_t *crows = nullptr);
   void to_fused(const double *canon, double *fused);
   void to_canonical(const double *fused, double *canon);
   void execute(const void *in0, const void *in1, void *out);
@@ -185,11 +188,12 @@ void launch_mpo_stage(int bm, int bn, bool cplx, bool f32, int out_planes, int64
 // FP64 vector) or stage 3 (A and B planes, FP64 output); FP64 -> 3 bf16 planes
 void launch_grouped_gemm_planar(int mode, int bm, int bn, bool stage3, const GemmTile *tiles, const GemmTask *tasks,
                                 const GemmSeg *segs, const Slots &slots, int ntiles, hipStream_t st);
-void launch_split_planes(const double *src, void *dst, int64_t n, hipStream_t st);
 void launch_grouped_gemm_mixed(int mode, int bm, int bn, bool b_f64, bool c_f64, bool cplx, const GemmTile *tiles,
                                const GemmTask *tasks, const GemmSeg *segs, const Slots &slots, int ntiles,
                                hipStream_t st);
-void launch_tile_trans(bool cplx, const TransDesc *d, int n, const double *src, double *dst, hipStream_t st);
+void launch_tile_trans(bool cplx, int out, const TransDesc *d, int n, const double *src, void *dst, int64_t ps,
+                       hipStream_t st);
+void split_copies(std::vector<CopyDesc> &v);
 void launch_f64_to_f32(const double *src, float *dst, int64_t n, hipStream_t st);
 void launch_block_copy(bool cplx, const CopyDesc *d, int n, const double *src, double *dst, hipStream_t st);
 void validate_stage(const Stage &s, const int64_t *slot_elems);
