@@ -1,0 +1,78 @@
+"""Small real symmetric matrices through ``qlg_eigh_batched``: orders around the
+in-LDS solver's thread counts and its upper limit (64; 65 and up run on the
+library's solver), odd orders, batches, and spectra that a Jacobi method can stumble
+over (graded Gram matrices, repeated and zero eigenvalues, diagonal and
+indefinite matrices).
+
+Bars: an orthogonal method's backward error is a modest multiple of n eps |A|;
+values and residuals are held to 4 n eps |A|_2, orthonormality to 8 n eps, with
+numpy's ``eigvalsh`` (itself n eps |A|) as the reference."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from ultradmrg_amd.sweep import eigh_batched
+
+EPS = np.finfo(float).eps
+KINDS = ["random", "graded", "rank", "diagonal", "zero", "repeated"]
+
+
+def _matrix(kind, n, rng):
+    if kind == "random":
+        a = rng.standard_normal((n, n))
+        return a + a.T
+    if kind == "graded":   # a unit-norm Gram matrix, singular values over 8 decades
+        x = (rng.standard_normal((n, n)) * 10.0 ** (-8.0 * np.arange(n) / n)) @ rng.standard_normal((n, 2 * n))
+        x /= np.linalg.norm(x)
+        return x @ x.T
+    if kind == "rank":
+        x = rng.standard_normal((n, max(1, n // 3)))
+        return x @ x.T
+    if kind == "diagonal":
+        return np.diag(rng.standard_normal(n))
+    if kind == "zero":
+        return np.zeros((n, n))
+    q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    return (q * np.where(np.arange(n) % 2, 2.0, -1.0)) @ q.T
+
+
+@pytest.mark.parametrize("n", [2, 3, 15, 16, 17, 24, 25, 33, 48, 49, 63, 64, 65, 97])
+def test_small_orders(n):
+    print(f"[case] order {n}", flush=True)
+    rng = np.random.default_rng(n)
+    mats = []
+    for k in KINDS:
+        a = _matrix(k, n, rng)
+        mats.append((a + a.T) / 2)
+    dev = torch.from_numpy(np.stack(mats)).cuda()
+    (w, v), = eigh_batched([dev.contiguous()])
+    w, v = w.cpu().numpy(), v.cpu().numpy()
+    for k, a, wi, vi in zip(KINDS, mats, w, v):
+        nrm = max(np.linalg.norm(a, 2), np.finfo(float).tiny)
+        assert np.all(np.diff(wi) >= 0), k
+        assert np.abs(wi - np.linalg.eigvalsh(a)).max() <= 4 * n * EPS * nrm, k
+        assert np.linalg.norm(a @ vi - vi * wi, 2) <= 4 * n * EPS * nrm, k
+        assert np.linalg.norm(vi.T @ vi - np.eye(n), 2) <= 8 * n * EPS, k
+
+
+def test_mixed_groups():
+    """Small and large orders in one call, and a non-finite input beside finite ones."""
+    print("[case] mixed groups", flush=True)
+    rng = np.random.default_rng(0)
+    groups = []
+    for n, b in ((16, 5), (64, 2), (130, 3), (40, 1)):
+        a = rng.standard_normal((b, n, n))
+        groups.append((a + a.transpose(0, 2, 1)) / 2)
+    groups[0][2, 3, 1] = np.nan
+    out = eigh_batched([torch.from_numpy(g.copy()).cuda() for g in groups])
+    for g, (w, v) in zip(groups, out):
+        w, v = w.cpu().numpy(), v.cpu().numpy()
+        for a, wi, vi in zip(g, w, v):
+            if not np.isfinite(a).all():
+                assert not np.isfinite(wi).any()
+                continue
+            n = a.shape[0]
+            assert np.linalg.norm(a @ vi - vi * wi, 2) <= 4 * n * EPS * np.linalg.norm(a, 2)

@@ -101,8 +101,14 @@ static void warm_up(EighPool &p) {
 
 static EighPool *pool(Ctx &c) {
   if (c.eig) return c.eig;
-  auto *p = new EighPool();
-  p->device = c.device;
+  c.eig = new EighPool();
+  c.eig->device = c.device;
+  return c.eig;
+}
+
+// the lanes' streams and handles, on the first batch that needs them
+static void make_lanes(EighPool *p) {
+  if (p->fork) return;
   try {
     for (auto &l : p->lane) {
       QLG_HIP(hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking));
@@ -115,11 +121,16 @@ static EighPool *pool(Ctx &c) {
     QLG_HIP(hipEventCreateWithFlags(&p->fork, hipEventDisableTiming));
     warm_up(*p);
   } catch (...) {
-    destroy_eigh_pool(p);
+    for (auto &l : p->lane) {
+      if (l.handle) (void)rocblas_destroy_handle(l.handle);
+      if (l.done) (void)hipEventDestroy(l.done);
+      if (l.stream) (void)hipStreamDestroy(l.stream);
+      l = Lane{};
+    }
+    if (p->fork) (void)hipEventDestroy(p->fork);
+    p->fork = nullptr;
     throw;
   }
-  c.eig = p;
-  return p;
 }
 
 static void solve_group(rocblas_handle h, int dtype, const qlg_eigh_group &g, double *e, int *info) {
@@ -169,8 +180,10 @@ void eigh_batched(Ctx &c, int dtype, int64_t ngroups, const qlg_eigh_group *grou
   }
   // longest-processing-time assignment; a group costs ~ its order (launch
   // latency per column) with a mild batch term
-  std::vector<int64_t> order(ngroups);
-  std::iota(order.begin(), order.end(), 0);
+  std::vector<int64_t> order, small;
+  for (int64_t k = 0; k < ngroups; ++k)
+    (dtype == QLG_F64 && groups[k].n <= kSmallEigh ? small : order).push_back(k);
+  if (!order.empty()) make_lanes(p);
   auto cost = [&](int64_t k) { return (double)groups[k].n * (1.0 + 0.05 * (double)groups[k].batch); };
   std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return cost(a) > cost(b); });
   std::vector<std::vector<int64_t>> work(kLanes);
@@ -186,7 +199,7 @@ void eigh_batched(Ctx &c, int dtype, int64_t ngroups, const qlg_eigh_group *grou
   const bool profile = prf && prf[0] == '1';
   double lane_ms[kLanes] = {0, 0, 0, 0};
   const auto t0 = std::chrono::steady_clock::now();
-  QLG_HIP(hipEventRecord(p->fork, c.stream));
+  if (!order.empty()) QLG_HIP(hipEventRecord(p->fork, c.stream));
   std::exception_ptr err[kLanes];
   std::vector<std::thread> th;
   for (int j = 0; j < kLanes; ++j) {
@@ -206,6 +219,15 @@ void eigh_batched(Ctx &c, int dtype, int64_t ngroups, const qlg_eigh_group *grou
         err[j] = std::current_exception();
       }
     });
+  }
+  // small orders on the context stream, beside the lanes (one launch a group)
+  std::exception_ptr small_err;
+  try {
+    for (int64_t k : small)
+      launch_jacobi_eigh(static_cast<double *>(groups[k].a), groups[k].w, info + i_off[k], (int)groups[k].n,
+                         (int)groups[k].batch, c.stream);
+  } catch (...) {
+    small_err = std::current_exception();
   }
   for (auto &t : th) t.join();
   if (profile) {
@@ -234,12 +256,16 @@ void eigh_batched(Ctx &c, int dtype, int64_t ngroups, const qlg_eigh_group *grou
     }
   for (int j = 0; j < kLanes; ++j)
     if (!work[j].empty()) QLG_HIP(hipStreamWaitEvent(c.stream, p->lane[j].done, 0));
+  if (small_err) {
+    (void)hipStreamSynchronize(c.stream);
+    std::rethrow_exception(small_err);
+  }
   QLG_HIP(hipMemcpyAsync(p->host_info, info, (size_t)ni * sizeof(int), hipMemcpyDeviceToHost, c.stream));
   QLG_HIP(hipStreamSynchronize(c.stream));
   for (int64_t k = 0; k < ngroups; ++k)
     for (int64_t i = 0; i < groups[k].batch; ++i)
       if (p->host_info[i_off[k] + i] != 0)
-        throw Error(QLG_ERR_NUMERIC, "eigh: divide-and-conquer did not converge (group " + std::to_string(k) +
+        throw Error(QLG_ERR_NUMERIC, "eigh: a decomposition did not converge (group " + std::to_string(k) +
                                          ", matrix " + std::to_string(i) + ", info " +
                                          std::to_string(p->host_info[i_off[k] + i]) + ")");
 }

@@ -1,0 +1,203 @@
+// Eigen-decompositions of small real symmetric matrices, one workgroup each,
+// entirely in LDS: the cyclic two-sided Jacobi method with the round-robin
+// ordering (every round rotates n / 2 disjoint pairs).
+//
+// The block SVD of a short chain, or of the edge sectors of a large one, has
+// Gram matrices of a few tens of rows.  The library's divide and conquer
+// spends several launches per column on them (0.6 ms of kernels and over 1 ms
+// of host time at order 32, whatever the batch); here a whole batch is one
+// launch.  A sweep of a 20-site chain at D = 48, whose 36 updates are mostly
+// such decompositions, went from 156 to 100 ms.  A round is bound by latency: the rotation angles (two reciprocals
+// and two reciprocal square roots in sequence), two barriers and the LDS round
+// trips between them; a matrix takes n - 1 rounds a sweep and 6 to 9 sweeps.
+//
+// A pair is rotated while |a_pq| > 4 eps sqrt(|a_pp a_qq|) and above 1e-3 eps
+// |A|_F: the Gram matrices' small eigenvalues keep their relative accuracy as
+// long as the matrix itself does.  A matrix whose pairs stay above that for
+// kSweeps sweeps (an indefinite one can, at rounding level) is accepted if its
+// off-diagonal elements are within 16 eps |A|_F.
+#include <hip/hip_runtime.h>
+
+#include "common.h"
+#include "eigh.h"
+
+namespace qlg {
+
+namespace {
+constexpr double kEps = 2.220446049250313e-16;
+constexpr int kSweeps = 24;
+
+// reciprocal and reciprocal square root from the hardware estimates and Newton
+// steps: a third of the latency of the IEEE sequences, which set a round's time
+__device__ inline double recip(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+__device__ inline double rsqrt_(double x) {
+  double r = __builtin_amdgcn_rsq(x);
+  r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
+  return fma(0.5 * r, fma(-x * r, r, 1.0), r);
+}
+
+__device__ inline double block_sum(double v, double *red) {
+  const int tid = threadIdx.x;
+  for (int o = 32; o; o >>= 1) v += __shfl_xor(v, o);
+  __syncthreads();
+  if ((tid & 63) == 0) red[tid >> 6] = v;
+  __syncthreads();
+  double s = 0.0;
+  for (int i = 0; i < (int)blockDim.x / 64; ++i) s += red[i];
+  return s;
+}
+}  // namespace
+
+// a: [batch][n][n] row-major symmetric; on return row j is eigenvector j, w
+// the ascending eigenvalues; info[m] = 0, or 1 if matrix m did not converge.
+// Dynamic LDS: A and V, [n][n + 1] doubles each.
+__global__ __launch_bounds__(1024) void jacobi_eigh_kernel(double *__restrict__ a, double *__restrict__ w, int *__restrict__ info, int n) {
+  extern __shared__ double lds[];
+  __shared__ double red[16];   // one per wave
+  __shared__ double cs[kSmallEigh / 2][2];
+  __shared__ int pk[kSmallEigh / 2], qk[kSmallEigh / 2];
+  __shared__ int rotated;
+  const int ld = n + 1, tid = threadIdx.x, nt = blockDim.x;
+  double *A = lds, *V = lds + n * ld;
+  double *ga = a + (int64_t)blockIdx.x * n * n;
+  double *gw = w + (int64_t)blockIdx.x * n;
+  double fro = 0.0;
+  for (int e = tid; e < n * n; e += nt) {
+    const int i = e / n, j = e % n;
+    // the lower triangle is the input, as for the library's solver
+    const double v = ga[i >= j ? e : j * n + i];
+    A[i * ld + j] = v;
+    V[i * ld + j] = i == j ? 1.0 : 0.0;
+    fro += v * v;
+  }
+  fro = sqrt(block_sum(fro, red));
+  if (!(fro < 1.0e300)) {   // NaN or infinity in the input: NaN out
+    for (int e = tid; e < n * n; e += nt) ga[e] = fro - fro;
+    for (int i = tid; i < n; i += nt) gw[i] = fro - fro;
+    if (tid == 0) info[blockIdx.x] = 0;
+    return;
+  }
+  // scaled by a power of two to a norm in [1, 2): no product below overflows,
+  // and no reciprocal meets a denormal number
+  int ex = 0;
+  if (fro > 0.0) {
+    ex = ilogb(fro);
+    fro = ldexp(fro, -ex);
+    for (int e = tid; e < n * n; e += nt) A[e / n * ld + e % n] = ldexp(A[e / n * ld + e % n], -ex);
+    __syncthreads();
+  }
+  const int np = (n + 1) & ~1, half = np / 2;   // odd n: one index sits out each round
+  const int lgh = half > 1 ? 32 - __clz(half - 1) : 0, lgn = n > 1 ? 32 - __clz(n - 1) : 0;
+  const double floor_abs = 1e-3 * kEps * fro;
+  int sweep = 0;
+  bool done = n < 2;
+  for (; !done && sweep < kSweeps; ++sweep) {
+    if (tid == 0) rotated = 0;
+    __syncthreads();
+    for (int r = 0; r < np - 1; ++r) {
+      // pair k of round r: position 0 is fixed, the others rotate by r
+      auto at = [&](int pos) { return pos == 0 ? 0 : 1 + (pos - 1 + r) % (np - 1); };
+      if (tid < half) {
+        int p = at(tid), q = at(np - 1 - tid);
+        if (p > q) {
+          const int t = p;
+          p = q;
+          q = t;
+        }
+        double c = 1.0, s = 0.0;
+        if (q < n) {
+          const double app = A[p * ld + p], aqq = A[q * ld + q], apq = A[p * ld + q], m = fabs(apq);
+          if (m > floor_abs && m > 4.0 * kEps * sqrt(fabs(app * aqq))) {
+            // tan of the smaller rotation angle; c is 1 / sqrt(1 + t^2) to the
+            // last bits, so that the rotation is orthogonal whatever t's error
+            const double th = (aqq - app) * recip(2.0 * apq), h = fabs(th);
+            const double y = 1.0 + th * th;
+            const double t0 = h > 1e8 ? 0.5 * recip(h) : recip(h + y * rsqrt_(y));
+            const double t = th >= 0.0 ? t0 : -t0;
+            c = rsqrt_(1.0 + t * t);
+            s = t * c;
+            rotated = 1;
+          }
+        }
+        cs[tid][0] = c;
+        cs[tid][1] = s;
+        pk[tid] = p;
+        qk[tid] = q;
+      }
+      __syncthreads();
+      // A <- J^T A J on 2 x 2 blocks (pair k's rows, pair l's columns), and
+      // rows p, q of V: one index space, so that every thread has an item
+      const int na = half << lgh, nv = half << lgn;
+      for (int e = tid; e < na + nv; e += nt) {
+        if (e >= na) {
+          const int k = (e - na) >> lgn, j = (e - na) & ((1 << lgn) - 1);
+          const double c = cs[k][0], s = cs[k][1];
+          if (s == 0.0 || j >= n) continue;
+          const int p = pk[k], q = qk[k];
+          const double x = V[p * ld + j], y = V[q * ld + j];
+          V[p * ld + j] = c * x - s * y;
+          V[q * ld + j] = s * x + c * y;
+          continue;
+        }
+        const int k = e >> lgh, l = e & ((1 << lgh) - 1);
+        if (l >= half) continue;
+        const double ck = cs[k][0], sk = cs[k][1], cl = cs[l][0], sl = cs[l][1];
+        if (sk == 0.0 && sl == 0.0) continue;
+        const int p = pk[k], q = qk[k], u = pk[l], v = qk[l];
+        const bool hq = q < n, hv = v < n;   // (an index that sits out has c = 1, s = 0)
+        const double x00 = A[p * ld + u], x01 = hv ? A[p * ld + v] : 0.0;
+        const double x10 = hq ? A[q * ld + u] : 0.0, x11 = hq && hv ? A[q * ld + v] : 0.0;
+        const double y00 = ck * x00 - sk * x10, y10 = sk * x00 + ck * x10;
+        const double y01 = ck * x01 - sk * x11, y11 = sk * x01 + ck * x11;
+        A[p * ld + u] = cl * y00 - sl * y01;
+        if (hv) A[p * ld + v] = k == l ? 0.0 : sl * y00 + cl * y01;
+        if (hq) A[q * ld + u] = k == l ? 0.0 : cl * y10 - sl * y11;
+        if (hq && hv) A[q * ld + v] = sl * y10 + cl * y11;
+      }
+      __syncthreads();
+    }
+    done = rotated == 0;
+    __syncthreads();
+  }
+  int bad = 0;
+  if (!done) {
+    double off = 0.0;
+    for (int e = tid; e < n * n; e += nt) {
+      const int i = e / n, j = e % n;
+      if (i != j) off += A[i * ld + j] * A[i * ld + j];
+    }
+    off = sqrt(block_sum(off, red));
+    bad = !(off <= 16.0 * kEps * fro);
+  }
+  if (tid == 0) info[blockIdx.x] = bad;
+  // ascending order: an eigenvalue's place is the number of smaller ones
+  for (int i = tid >> 6; i < n; i += nt >> 6) {
+    const double x = A[i * ld + i];
+    int rank = 0;
+    for (int j0 = 0; j0 < n; j0 += 64) {
+      const int j = j0 + (tid & 63);
+      const double y = j < n ? A[j * ld + j] : 0.0;
+      rank += __popcll(__ballot(j < n && (y < x || (y == x && j < i))));
+    }
+    if ((tid & 63) == 0) gw[rank] = ldexp(x, ex);
+    for (int j = tid & 63; j < n; j += 64) ga[rank * n + j] = V[i * ld + j];
+  }
+}
+
+void launch_jacobi_eigh(double *a, double *w, int *info, int n, int batch, hipStream_t st) {
+  QLG_CHECK(n >= 1 && n <= kSmallEigh, "small eigensolver: order out of range");
+  const size_t lds = (size_t)2 * n * (n + 1) * sizeof(double);
+  QLG_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(jacobi_eigh_kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              2 * kSmallEigh * (kSmallEigh + 1) * (int)sizeof(double)));
+  // a thread per 2 x 2 block of A and pair of V's elements, up to 1024
+  const int threads = n <= 16 ? 192 : n <= 24 ? 512 : 1024;
+  hipLaunchKernelGGL(jacobi_eigh_kernel, dim3(batch), dim3(threads), lds, st, a, w, info, n);
+  QLG_HIP(hipGetLastError());
+}
+
+}  // namespace qlg

@@ -65,7 +65,13 @@ struct Bucket {
   int64_t xbase = 0, gbase = 0, rbase = 0;
 };
 
-int64_t bucket_bound(int64_t n) {
+// Orders up to kSmallEigh are solved in LDS, a real bucket per launch, and gain from
+// buckets of their own; a complex one is a divide-and-conquer call whose time
+// is its largest order's, so small complex sectors share the first large one.
+int64_t bucket_bound(int64_t n, bool cplx) {
+  if (!cplx)
+    for (int64_t b : {int64_t(1), int64_t(16), int64_t(32), int64_t(48), int64_t(kSmallEigh)})
+      if (n <= b) return b;
   static const int64_t bounds[] = {1, 256, 512, 768, 1024, 1536, 2048, 3072, 4096, 6144, 8192};
   for (int64_t b : bounds)
     if (n <= b) return b;
@@ -240,7 +246,7 @@ SvdResult *block_svd(Ctx &c, const qlg_bsten *desc, int ldims, const int32_t *ld
   }
   // ---- buckets ------------------------------------------------------------------------
   std::map<int64_t, std::vector<int>> raw;
-  for (int s : order) raw[bucket_bound(sec[s].n)].push_back(s);
+  for (int s : order) raw[bucket_bound(sec[s].n, cplx)].push_back(s);
   std::vector<Bucket> bk;
   int64_t xtot = 0, gtot = 0, rtot = 0, nsv = 0;
   for (auto &kv : raw) {
