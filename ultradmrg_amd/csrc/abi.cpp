@@ -311,7 +311,7 @@ int qlg_plan_workspace(qlg_plan plan, int64_t *bytes) {
   if (!plan || !bytes) return QLG_ERR_INVALID;
   Plan &p = *plan->p;
   int64_t b = (int64_t)(p.X.bytes + p.Y.bytes + p.C.bytes + p.basis.bytes);
-  for (auto &s : p.st) b += (int64_t)(s.d_tiles.bytes + s.d_tasks.bytes + s.d_segs.bytes);
+  for (int i = 0; i < 3; ++i) b += (int64_t)(p.st[i].lists.bytes + p.rst[i].lists.bytes);
   *bytes = b;
   return QLG_OK;
 }

@@ -302,12 +302,19 @@ void Stage::find_direct() {
 }
 
 void Stage::upload(hipStream_t st) {
+  std::vector<char> &host = staged;
+  host.clear();
+  std::vector<std::pair<DevList *, size_t>> parts;
+  auto add = [&](DevList &d, const auto &v) {
+    d.p = nullptr;
+    if (v.empty()) return;
+    host.resize((host.size() + 63) / 64 * 64);
+    parts.push_back({&d, host.size()});
+    const char *src = reinterpret_cast<const char *>(v.data());
+    host.insert(host.end(), src, src + v.size() * sizeof(v[0]));
+  };
   if (!chan.empty()) {
-    d_chan.ensure(chan.size() * sizeof(ChanTask));
-    d_rows.ensure(std::max<size_t>(1, rows.size()) * sizeof(RowDesc));
-    QLG_HIP(hipMemcpyAsync(d_chan.p, chan.data(), chan.size() * sizeof(ChanTask), hipMemcpyHostToDevice, st));
-    if (!rows.empty())
-      QLG_HIP(hipMemcpyAsync(d_rows.p, rows.data(), rows.size() * sizeof(RowDesc), hipMemcpyHostToDevice, st));
+    add(d_rows, rows);
     ctiles.assign(tiles.size(), ChanTile{});
     for (size_t i = 0; i < tiles.size(); ++i) {
       const GemmTile &t = tiles[i];
@@ -321,33 +328,23 @@ void Stage::upload(hipStream_t st) {
       o.m0 = t.m0;
       o.n0 = t.n0;
     }
-    d_ctiles.ensure(std::max<size_t>(1, ctiles.size()) * sizeof(ChanTile));
-    if (!ctiles.empty())
-      QLG_HIP(hipMemcpyAsync(d_ctiles.p, ctiles.data(), ctiles.size() * sizeof(ChanTile), hipMemcpyHostToDevice, st));
+    add(d_ctiles, ctiles);
+  } else {
+    // the split lists when a task is split
+    add(d_crows, crows);
+    add(d_tiles, tiles);
+    add(d_tasks, split() ? ktasks : tasks);
+    add(d_segs, split() ? ksegs : segs);
+    if (split()) {
+      add(d_red, red);
+      add(d_redc, redc);
+      work.ensure((size_t)std::max<int64_t>(work_elems, 1) * ed * sizeof(double));
+    }
   }
-  if (!crows.empty()) {
-    d_crows.ensure(crows.size() * sizeof(int64_t));
-    QLG_HIP(hipMemcpyAsync(d_crows.p, crows.data(), crows.size() * sizeof(int64_t), hipMemcpyHostToDevice, st));
-  }
-  // the launch lists: the split ones when a task is split
-  const std::vector<GemmTask> &lt = split() ? ktasks : tasks;
-  const std::vector<GemmSeg> &ls = split() ? ksegs : segs;
-  d_tiles.ensure(std::max<size_t>(1, tiles.size()) * sizeof(GemmTile));
-  d_tasks.ensure(std::max<size_t>(1, lt.size()) * sizeof(GemmTask));
-  d_segs.ensure(std::max<size_t>(1, ls.size()) * sizeof(GemmSeg));
-  if (!tiles.empty())
-    QLG_HIP(hipMemcpyAsync(d_tiles.p, tiles.data(), tiles.size() * sizeof(GemmTile), hipMemcpyHostToDevice, st));
-  if (!lt.empty())
-    QLG_HIP(hipMemcpyAsync(d_tasks.p, lt.data(), lt.size() * sizeof(GemmTask), hipMemcpyHostToDevice, st));
-  if (!ls.empty())
-    QLG_HIP(hipMemcpyAsync(d_segs.p, ls.data(), ls.size() * sizeof(GemmSeg), hipMemcpyHostToDevice, st));
-  if (split()) {
-    d_red.ensure(red.size() * sizeof(RedTask));
-    d_redc.ensure(redc.size() * sizeof(RedChunk));
-    work.ensure((size_t)std::max<int64_t>(work_elems, 1) * ed * sizeof(double));
-    QLG_HIP(hipMemcpyAsync(d_red.p, red.data(), red.size() * sizeof(RedTask), hipMemcpyHostToDevice, st));
-    QLG_HIP(hipMemcpyAsync(d_redc.p, redc.data(), redc.size() * sizeof(RedChunk), hipMemcpyHostToDevice, st));
-  }
+  if (host.empty()) return;
+  lists.ensure(host.size());
+  for (auto &pt : parts) pt.first->p = lists.as<char>() + pt.second;
+  QLG_HIP(hipMemcpyAsync(lists.p, host.data(), host.size(), hipMemcpyHostToDevice, st));
 }
 
 // Bounds of every access a task list can make: rows < M, cols < N, k < K of

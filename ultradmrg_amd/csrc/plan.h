@@ -25,7 +25,16 @@ struct Stage {
   std::vector<ChanTask> chan;      // MPO-stage channels (instead of tasks)
   std::vector<RowDesc> rows;       // their gathered / scattered rows
   std::vector<ChanTile> ctiles;    // MPO stage: tiles with their channels inlined (upload)
-  DevBuf d_tiles, d_tasks, d_segs, d_crows, d_chan, d_rows, d_ctiles;
+  // device copies of the launch lists: parts of one buffer, filled by one copy
+  // (a copy of a few hundred bytes costs the host as much as a launch, and a
+  // sweep of a short chain made 130 of them per update)
+  struct DevList {
+    void *p = nullptr;
+    template <class T> T *as() const { return static_cast<T *>(p); }
+  };
+  DevBuf lists;
+  std::vector<char> staged;
+  DevList d_tiles, d_tasks, d_segs, d_crows, d_rows, d_ctiles, d_red, d_redc;
   int bm = 64, bn = 64;
   double flops = 0;      // useful 2*M*N*K issued by this stage
   double algo_flops = 0; // this stage's share of the reference schedule's FLOPs
@@ -46,7 +55,7 @@ struct Stage {
   std::vector<RedTask> red;
   std::vector<RedChunk> redc;
   int64_t work_elems = 0;
-  DevBuf d_red, d_redc, work;
+  DevBuf work;
   void upload(hipStream_t st);
   void make_tiles(int bm_, int bn_);
   bool split() const { return kchunk > 0 && !red.empty(); }

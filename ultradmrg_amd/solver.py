@@ -29,7 +29,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
-from .tensor import BlockTensor, Context, default_context
+from .tensor import BlockTensor, Context, default_context, layout_lists
 
 PRECISIONS = {"fp64": L.QLG_PREC_F64, "fp32": L.QLG_PREC_F32, "bf16x3": L.QLG_PREC_BF16X3,
               "bf16x6": L.QLG_PREC_BF16X6}
@@ -112,12 +112,8 @@ class EffectiveHamiltonian:
         self.lib = lib
         nb, size = C.c_int64(), C.c_int64()
         self.ctx.check(lib.qlg_plan_vector_layout(h, C.byref(nb), C.byref(size), None, None))
-        coords = (C.c_int32 * max(nb.value * state.rank, 1))()
-        offs = (C.c_int64 * max(nb.value, 1))()
-        self.ctx.check(lib.qlg_plan_vector_layout(h, None, None, coords, offs))
-        r = state.rank
-        self.layout_coords = [tuple(coords[b * r:(b + 1) * r]) for b in range(nb.value)]
-        self.layout_offsets = list(offs[:nb.value])
+        self.layout_coords, self.layout_offsets = layout_lists(
+            nb.value, state.rank, lambda c, o: self.ctx.check(lib.qlg_plan_vector_layout(h, None, None, c, o)))
         self.size = size.value
         self.axes = state.axes
         self.dtype = state.data.dtype
@@ -126,7 +122,7 @@ class EffectiveHamiltonian:
     # ----- layout helpers ------------------------------------------------------------
     def new_vector(self, zero=True) -> BlockTensor:
         buf = (torch.zeros if zero else torch.empty)(max(self.size, 1), dtype=self.dtype, device=self.device)
-        return BlockTensor(self.axes, self.layout_coords, buf, self.layout_offsets)
+        return BlockTensor._on_layout(self.axes, self.layout_coords, self.layout_offsets, self.size, buf)
 
     def adopt(self, state: BlockTensor) -> BlockTensor:
         """Return ``state`` in the plan's Krylov layout (copying blocks if the layouts differ).
@@ -277,7 +273,8 @@ class BatchedEffectiveHamiltonian:
     def unpack(self, buf: torch.Tensor) -> List[BlockTensor]:
         out = []
         for m, o in zip(self.members, self.offsets):
-            out.append(BlockTensor(m.axes, m.layout_coords, buf[o:o + max(m.size, 1)].clone(), m.layout_offsets))
+            out.append(BlockTensor._on_layout(m.axes, m.layout_coords, m.layout_offsets, m.size,
+                                             buf[o:o + max(m.size, 1)].clone()))
         return out
 
     def flops(self):

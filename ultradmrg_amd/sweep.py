@@ -30,7 +30,7 @@ import torch
 from .mpo import Model, physical_axis
 from .solver import EffectiveHamiltonian, LanczosParams
 from . import _lib as L
-from .tensor import IN, OUT, Axis, BlockTensor, _flow, contract, default_context, env_update
+from .tensor import IN, OUT, Axis, BlockTensor, _flow, contract, default_context, env_update, layout_lists
 
 
 def divergence(t: BlockTensor) -> Tuple[int, ...]:
@@ -111,16 +111,14 @@ def block_svd(t: BlockTensor, ldims: int, ldiv, trunc_err: float, Dmin: int, Dma
             nb, size = C.c_int64(), C.c_int64()
             ctx.check(lib.qlg_svd_tensor(h, which, C.byref(nb), C.byref(size), None, None, None))
             r = len(axes)
-            coords = (C.c_int32 * max(nb.value * r, 1))()
-            offs = (C.c_int64 * max(nb.value, 1))()
             data = C.c_void_p()
-            ctx.check(lib.qlg_svd_tensor(h, which, None, None, coords, offs, C.byref(data)))
+            cl, offs = layout_lists(
+                nb.value, r, lambda co, of: ctx.check(lib.qlg_svd_tensor(h, which, None, None, co, of, C.byref(data))))
             buf = torch.empty(max(size.value, 1), dtype=dtype, device=dev)
             nbytes = size.value * buf.element_size()
             if nbytes:
                 ctx.check(lib.qlg_memcpy_d2d(ctx.h, C.c_void_p(buf.data_ptr()), data, nbytes))
-            cl = [tuple(coords[b * r:(b + 1) * r]) for b in range(nb.value)]
-            return BlockTensor(axes, cl, buf, list(offs[:nb.value]))
+            return BlockTensor._on_layout(axes, cl, offs, size.value, buf)
 
         dt = t.data.dtype
         u = fetch(0, list(t.axes[:ldims]) + [mid_out], dt)
@@ -128,10 +126,8 @@ def block_svd(t: BlockTensor, ldims: int, ldiv, trunc_err: float, Dmin: int, Dma
         vt = fetch(2, [mid_in] + list(t.axes[ldims:]), dt)
     finally:
         lib.qlg_svd_destroy(h)
-    # kept singular values: the diagonals of s's blocks
-    diag = torch.cat([s.data[o:o + k * k].view(k, k).diagonal()
-                      for (mi, _), o, k in zip(s.coords, s.offsets, mid_out.degs)]) if s.coords else s.data[:0]
-    pr = diag.double() ** 2
+    # s holds the kept singular values on its blocks' diagonals, zeros elsewhere
+    pr = s.data.double() ** 2
     pr = pr / pr.sum() if float(pr.sum()) > 0 else pr
     pr = pr[pr > 0]
     ee = float(-(pr * torch.log(pr)).sum()) if pr.numel() else 0.0

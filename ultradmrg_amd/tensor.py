@@ -11,6 +11,7 @@ descriptor handed to the library is zero-copy.
 from __future__ import annotations
 
 import ctypes as C
+from itertools import chain
 from dataclasses import dataclass
 from typing import Dict, Optional, Sequence, Tuple
 
@@ -58,16 +59,35 @@ class BlockTensor:
     def __init__(self, axes: Sequence[Axis], coords: Sequence[Tuple[int, ...]], data: torch.Tensor,
                  offsets: Optional[Sequence[int]] = None):
         self.axes = list(axes)
-        self.coords = [tuple(int(v) for v in c) for c in coords]
-        sizes = [self.block_size(c) for c in self.coords]
+        # whole-array bookkeeping: a two-site tensor has hundreds of blocks, and a
+        # Python loop over them costs more than the contraction that made it
+        coords = list(coords)
+        ints = np.fromiter(chain.from_iterable(coords), dtype=np.int64)
+        ints = ints.reshape(len(coords), -1 if coords else len(self.axes))
+        self.coords = list(map(tuple, ints.tolist()))
+        sizes = np.ones(len(ints), dtype=np.int64)
+        for ax, col in zip(self.axes, ints.T):
+            sizes *= np.array(ax.degs, dtype=np.int64)[col]
         if offsets is None:
-            offsets = np.concatenate([[0], np.cumsum(sizes)[:-1]]).astype(np.int64) if sizes else []
-        self.offsets = [int(o) for o in offsets]
-        self.size = int(max([o + s for o, s in zip(self.offsets, sizes)], default=0))
+            offsets = np.cumsum(sizes) - sizes
+        offs = np.array(offsets, dtype=np.int64).reshape(-1)
+        self.offsets = offs.tolist()
+        n = min(len(offs), len(sizes))
+        self.size = int((offs[:n] + sizes[:n]).max()) if n else 0
         if data.numel() < self.size:
             raise ValueError("data buffer smaller than the block layout")
         self.data = data
         self._desc_keep = None
+
+    @classmethod
+    def _on_layout(cls, axes: Sequence[Axis], coords, offsets, size: int, data: torch.Tensor) -> "BlockTensor":
+        """A tensor on a layout that the library gave (lists of ints, checked there)."""
+        t = cls.__new__(cls)
+        t.axes, t.coords, t.offsets, t.size = list(axes), list(coords), list(offsets), size
+        if data.numel() < size:
+            raise ValueError("data buffer smaller than the block layout")
+        t.data, t._desc_keep = data, None
+        return t
 
     # ----- structure ------------------------------------------------------------
     @property
@@ -121,12 +141,13 @@ class BlockTensor:
         degs = [d for ax in self.axes for d in ax.degs]
         sect_deg = (C.c_int64 * max(len(degs), 1))(*degs)
         dirs = (C.c_int8 * r)(*[ax.dir for ax in self.axes])
-        flat = [v for c in self.coords for v in c]
-        coords = (C.c_int32 * max(len(flat), 1))(*flat)
-        offs = (C.c_int64 * max(len(self.offsets), 1))(*self.offsets)
-        d = L.Bsten(r, self.qn_len, nsect, sect_qn, sect_deg, dirs, len(self.coords), coords, offs,
+        flat = np.fromiter(chain.from_iterable(self.coords or [(0,)]), dtype=np.int32)
+        offs = np.array(self.offsets or [0], dtype=np.int64)
+        coords = flat.ctypes.data_as(C.POINTER(C.c_int32))
+        d = L.Bsten(r, self.qn_len, nsect, sect_qn, sect_deg, dirs, len(self.coords), coords,
+                    offs.ctypes.data_as(C.POINTER(C.c_int64)),
                     L.QLG_C128 if self.is_complex else L.QLG_F64, C.c_void_p(self.data.data_ptr()))
-        self._desc_keep = (nsect, sect_qn, sect_deg, dirs, coords, offs, d)
+        self._desc_keep = (nsect, sect_qn, sect_deg, dirs, flat, offs, d)
         return d
 
 
@@ -243,6 +264,14 @@ def linear_combine(coefs, bases: Sequence[torch.Tensor], beta, y: torch.Tensor, 
 # ---------------------------------------------------------------------------
 # contractions around the Krylov solve
 # ---------------------------------------------------------------------------
+def layout_lists(nb: int, rank: int, fill):
+    """Block coordinates (tuples) and offsets of a layout that ``fill(coords, offsets)`` writes."""
+    coords = np.zeros((max(nb, 1), rank), dtype=np.int32)
+    offs = np.zeros(max(nb, 1), dtype=np.int64)
+    fill(coords.ctypes.data_as(C.POINTER(C.c_int32)), offs.ctypes.data_as(C.POINTER(C.c_int64)))
+    return list(map(tuple, coords[:nb].tolist())), offs[:nb].tolist()
+
+
 class _OpPlan:
     """A tensordot / environment-update plan and its result layout."""
 
@@ -251,11 +280,8 @@ class _OpPlan:
         lib = ctx.lib
         nb, size = C.c_int64(), C.c_int64()
         ctx.check(lib.qlg_plan_vector_layout(handle, C.byref(nb), C.byref(size), None, None))
-        coords = (C.c_int32 * max(nb.value * rank, 1))()
-        offs = (C.c_int64 * max(nb.value, 1))()
-        ctx.check(lib.qlg_plan_vector_layout(handle, None, None, coords, offs))
-        self.coords = [tuple(coords[b * rank:(b + 1) * rank]) for b in range(nb.value)]
-        self.offsets = list(offs[:nb.value])
+        self.coords, self.offsets = layout_lists(
+            nb.value, rank, lambda c, o: ctx.check(lib.qlg_plan_vector_layout(handle, None, None, c, o)))
         self.size = size.value
 
     def run(self, in0: BlockTensor, in1: BlockTensor, dtype) -> BlockTensor:
@@ -263,7 +289,7 @@ class _OpPlan:
         self.ctx.check(self.ctx.lib.qlg_execute(self.h, C.c_void_p(in0.data.data_ptr()),
                                                 C.c_void_p(in1.data.data_ptr()), C.c_void_p(out.data_ptr())))
         self.ctx.synchronize()
-        return BlockTensor(self.axes, self.coords, out, self.offsets)
+        return BlockTensor._on_layout(self.axes, self.coords, self.offsets, self.size, out)
 
     def __del__(self):
         try:
