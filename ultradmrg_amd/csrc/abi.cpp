@@ -74,7 +74,7 @@ int qlg_ctx_create(int device, void *stream, qlg_ctx *out) {
       QLG_HIP(hipStreamCreateWithFlags(&h->c.stream, hipStreamNonBlocking));
       h->c.own_stream = true;
     }
-    h->c.partials.ensure(2 * kMaxPartials * sizeof(double));
+    h->c.partials.ensure(3 * kMaxPartials * sizeof(double));   // a step's dot (complex) and norm
     h->c.scalars.ensure(64 * sizeof(double));
     noalloc_init(device);   // address of the fixed staging array on this device
     QLG_HIP(hipHostMalloc((void **)&h->c.host_scalars, 64 * sizeof(double), hipHostMallocDefault));

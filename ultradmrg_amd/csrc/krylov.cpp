@@ -537,11 +537,14 @@ struct RunAhead {
       b[i] = p.host_lz[2 * i + 1];
     }
   }
-  // residual of iteration m in slot m+1 is final: reorthogonalise it and
-  // replace b_m by its norm
-  void reorth(int64_t m, const int *skip) {
+  // a_m and the residual of iteration m in slot m + 1; its norm b_m is left as
+  // partial sums for the check (or, after reorthogonalisation, written to b_m)
+  PartialNorm step(int64_t m, const int *skip) {
+    const PartialNorm nm = vec_lanczos_step(*p.ctx, p.dtype, w.n, w.slot(m + 1), w.slot(m), A(m),
+                                            m > 0 ? w.slot(m - 1) : nullptr, m > 0 ? B(m - 1) : nullptr, skip);
     for (int pass = 0; pass < p.reorth; ++pass)
       lz_reorth(p.ctx->stream, p.dtype, w.n, ptrs, (int)(m + 1), w.slot(m + 1), rpart, rc, B(m), skip);
+    return p.reorth > 0 ? PartialNorm{} : nm;
   }
   // queue iterations [m0, m1) with `body`, as a captured graph when the plan
   // uses graphs (one graph per chunk index, replayed by later solves with the
@@ -626,19 +629,14 @@ void lanczos_gs(Plan &p, double *psi, const qlg_lanczos_params &prm, qlg_lanczos
   p.matvec_fused(w.slot(0), w.slot(1));   // also settles the tile shapes before any capture
   {
     SkipGuard sg(p, &r.ctl->stop);
-    vec_dot(c, p.dtype, w.n, w.slot(1), w.slot(0), r.A(0), &r.ctl->stop);
-    vec_lanczos_residual(c, p.dtype, w.n, w.slot(1), w.slot(0), r.A(0), nullptr, nullptr, r.B(0), &r.ctl->stop);
-    r.reorth(0, &r.ctl->stop);
-    lz_gs_check(st, r.ab, r.ctl, 0, dim, maxit, prm.error);
+    const PartialNorm nm0 = r.step(0, &r.ctl->stop);
+    lz_gs_check(st, r.ab, nm0, r.ctl, 0, dim, maxit, prm.error);
     auto body = [&](int64_t m) {
       const int *skip = &r.ctl->stop;
       vec_scal_inv_dev(c, p.dtype, w.n, r.B(m - 1), w.slot(m), skip);
       p.matvec_fused(w.slot(m), w.slot(m + 1));
-      vec_dot(c, p.dtype, w.n, w.slot(m + 1), w.slot(m), r.A(m), skip);
-      vec_lanczos_residual(c, p.dtype, w.n, w.slot(m + 1), w.slot(m), r.A(m), w.slot(m - 1), r.B(m - 1), r.B(m),
-                           skip);
-      r.reorth(m, skip);
-      lz_gs_check(st, r.ab, r.ctl, (int)m, dim, maxit, prm.error);
+      const PartialNorm nm = r.step(m, skip);
+      lz_gs_check(st, r.ab, nm, r.ctl, (int)m, dim, maxit, prm.error);
     };
     const int64_t K = chunk_iterations();
     const std::string key = graph_key(r, "gs", prm.error, 0.0);
@@ -689,20 +687,15 @@ void lanczos_expmv(Plan &p, double *psi, double tau, const qlg_lanczos_params &p
   {
     SkipGuard sg(p, &r.ctl->stop);
     // a_m = Re <H v_m | v_m>: the complex dot writes (re, im) over (a_m, b_m);
-    // the residual reads the real part and then overwrites b_m with its norm
-    vec_dot(c, p.dtype, w.n, w.slot(1), w.slot(0), r.A(0), &r.ctl->stop);
-    vec_lanczos_residual(c, p.dtype, w.n, w.slot(1), w.slot(0), r.A(0), nullptr, nullptr, r.B(0), &r.ctl->stop);
-    r.reorth(0, &r.ctl->stop);
-    lz_expmv_check(st, r.ab, r.ctl, r.coef_cur, r.coef_prev, nullptr, 0, dim, maxit, prm.error, tau);
+    // the step uses the real part, and b_m is overwritten with the residual's norm
+    const PartialNorm nm0 = r.step(0, &r.ctl->stop);
+    lz_expmv_check(st, r.ab, nm0, r.ctl, r.coef_cur, r.coef_prev, 0, dim, maxit, prm.error, tau);
     auto body = [&](int64_t m) {
       const int *skip = &r.ctl->stop;
       vec_scal_inv_dev(c, p.dtype, w.n, r.B(m - 1), w.slot(m), skip);
       p.matvec_fused(w.slot(m), w.slot(m + 1));
-      vec_dot(c, p.dtype, w.n, w.slot(m + 1), w.slot(m), r.A(m), skip);
-      vec_lanczos_residual(c, p.dtype, w.n, w.slot(m + 1), w.slot(m), r.A(m), w.slot(m - 1), r.B(m - 1), r.B(m),
-                           skip);
-      r.reorth(m, skip);
-      lz_expmv_check(st, r.ab, r.ctl, r.coef_cur, r.coef_prev, nullptr, (int)m, dim, maxit, prm.error, tau);
+      const PartialNorm nm = r.step(m, skip);
+      lz_expmv_check(st, r.ab, nm, r.ctl, r.coef_cur, r.coef_prev, (int)m, dim, maxit, prm.error, tau);
     };
     const int64_t K = chunk_iterations();
     const std::string key = graph_key(r, "expmv", prm.error, tau);

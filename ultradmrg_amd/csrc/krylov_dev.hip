@@ -47,27 +47,73 @@ __global__ void lz_reset_kernel(LzCtl *ctl) {
   }
 }
 
+// Both checks are serial chains on one wave, so their time is the latency of
+// their divisions and square roots: these come from the hardware estimates and
+// two Newton steps (within an ulp or two), a third of the IEEE sequences'
+// latency.  Arguments stay far from the range's ends (see the callers).
+__device__ inline double recip(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+__device__ inline double rsqrt_(double x) {
+  double r = __builtin_amdgcn_rsq(x);
+  r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
+  return fma(0.5 * r, fma(-x * r, r, 1.0), r);
+}
+
+// sqrt of the sum of a step's partial sums, in the order of
+// reduce_partials_kernel (256 threads: lane l stands for threads l + 64 w)
+__device__ inline double partial_norm(PartialNorm p) {
+  const int lane = threadIdx.x;
+  double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+  for (int i = lane; i < p.count; i += 256)
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      if (i + 64 * w < p.count) v[w] += p.part[i + 64 * w];
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) v[w] += __shfl_xor(v[w], o, 64);
+  double s = 0.0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) s += v[w];
+  return sqrt(s);
+}
+
+// lane i's value of v, for an i that is the same in all lanes (a register
+// move; an LDS read is a hundred cycles in a serial chain)
+__device__ inline double lane_value(double v, int i) {
+  typedef int i2 __attribute__((ext_vector_type(2)));
+  const i2 b = __builtin_bit_cast(i2, v);
+  const i2 r = {__builtin_amdgcn_readlane(b.x, i), __builtin_amdgcn_readlane(b.y, i)};
+  return __builtin_bit_cast(double, r);
+}
+
 // number of eigenvalues of T below x (Sturm count), with the pivot guard of
 // LAPACK's dstebz
 __device__ inline int sturm_count(const double *a, const double *b2, int n, double x, double pivmin) {
   double q = a[0] - x;
   if (fabs(q) < pivmin) q = -pivmin;
   int c = q < 0.0 ? 1 : 0;
+#pragma unroll 4   // the next elements' LDS reads beside the division chain
   for (int i = 1; i < n; ++i) {
-    q = (a[i] - x) - b2[i - 1] / q;
+    q = (a[i] - x) - b2[i - 1] * recip(q);
     if (fabs(q) < pivmin) q = -pivmin;
     c += q < 0.0 ? 1 : 0;
   }
   return c;
 }
 
-__global__ __launch_bounds__(64) void lz_gs_check_kernel(const double *__restrict__ ab, LzCtl *ctl, int m,
+__global__ __launch_bounds__(64) void lz_gs_check_kernel(double *ab, PartialNorm norm, LzCtl *ctl, int m,
                                                          int64_t dim, int64_t maxit, double err) {
   if (ctl->stop) return;
   __shared__ double a[kMaxGsDim], b2[kMaxGsDim];
   const int lane = threadIdx.x;
   const int n = m + 1;
-  const double bm = ab[2 * m + 1];   // norm of the residual of this iteration
+  // norm of the residual of this iteration
+  const double bm = norm.part ? partial_norm(norm) : ab[2 * m + 1];
+  if (norm.part && lane == 0) ab[2 * m + 1] = bm;
   if (m == 0) {
     if (lane == 0) {
       ctl->e_prev = ab[0];
@@ -96,7 +142,8 @@ __global__ __launch_bounds__(64) void lz_gs_check_kernel(const double *__restric
     hi = fmax(hi, __shfl_xor(hi, o, 64));
   }
   __syncthreads();
-  const double pivmin = DBL_MIN * fmax(1.0, bmax2);
+  // far below the last bit of T, and large enough for recip(q) b^2 to stay finite
+  const double pivmin = fmax(DBL_MIN * fmax(1.0, bmax2), 1e-60 * fmax(fabs(lo), fabs(hi)));
   const double pad = 2.0 * DBL_EPSILON * fmax(fabs(lo), fabs(hi)) + pivmin;
   lo -= pad;
   hi += pad;
@@ -132,18 +179,19 @@ __global__ __launch_bounds__(64) void lz_gs_check_kernel(const double *__restric
   }
 }
 
-__global__ __launch_bounds__(64) void lz_expmv_check_kernel(const double *__restrict__ ab, LzCtl *ctl,
+__global__ __launch_bounds__(64) void lz_expmv_check_kernel(double *ab, PartialNorm norm, LzCtl *ctl,
                                                             double *__restrict__ cur, double *__restrict__ prev,
                                                             int m, int64_t dim, int64_t maxit, double err,
                                                             double tau) {
   if (ctl->stop) return;
   __shared__ double z[kZ * kZ];
-  __shared__ double d[kZ], e[kZ], tr[kZ], ti[kZ];
+  __shared__ double dsh[kZ], tr[kZ], ti[kZ];
   __shared__ int perm[kZ];
   const int lane = threadIdx.x;
   const int n = m + 1;
   const int ncoef = 2 * (int)(maxit + 1);
-  const double bm = ab[2 * m + 1];
+  const double bm = norm.part ? partial_norm(norm) : ab[2 * m + 1];
+  if (norm.part && lane == 0) ab[2 * m + 1] = bm;
   if (m == 0) {
     // coefficients of the breakdown case exp(-i tau a_0) e_1; the previous
     // coefficients start as zeros
@@ -161,72 +209,74 @@ __global__ __launch_bounds__(64) void lz_expmv_check_kernel(const double *__rest
     }
     return;
   }
-  // T_{m+1}: diagonal a_0..a_m, off-diagonal b_0..b_{m-1}
-  if (lane < n) {
-    d[lane] = ab[2 * lane];
-    e[lane] = lane + 1 < n ? ab[2 * lane + 1] : 0.0;
+  // T_{m+1}: diagonal a_0..a_m, off-diagonal b_0..b_{m-1}, scaled by a power of
+  // two to a largest element in [1, 2) so that sums of squares neither overflow
+  // nor lose what matters
+  int ex = 0;
+  // lane l holds d_l and e_l; the scalar recurrence runs on all lanes alike
+  double d = lane < n ? ab[2 * lane] : 0.0, e = lane + 1 < n ? ab[2 * lane + 1] : 0.0;
+  {
+    double big = fmax(fabs(d), fabs(e));
+    for (int o = 32; o > 0; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
+    if (big > 0.0 && big < DBL_MAX) ex = ilogb(big);
+    d = ldexp(d, -ex);
+    e = ldexp(e, -ex);
   }
-  for (int k = lane; k < n * n; k += 64) z[k] = (k / n == k % n) ? 1.0 : 0.0;
-  __syncthreads();
-  // implicit QL (tql2); every lane runs the scalar recurrence on the shared
-  // d and e, lane k < n applies the rotations to row k of z
+  for (int k = 0; k < n; ++k)
+    if (lane < n) z[lane * n + k] = k == lane ? 1.0 : 0.0;
+  // implicit QL (tql2); lane k < n applies the rotations to its own row k of z
   bool ok = true;
   for (int l = 0; l < n && ok; ++l) {
     int iter = 0;
     while (true) {
-      int mm = l;
-      for (; mm < n - 1; ++mm) {
-        const double dd = fabs(d[mm]) + fabs(d[mm + 1]);
-        if (fabs(e[mm]) <= DBL_EPSILON * dd) break;
-      }
+      // first negligible off-diagonal element at or after l
+      const double dn = __shfl_down(d, 1, 64);
+      const unsigned long long small =
+          __ballot(lane >= n - 1 || fabs(e) <= DBL_EPSILON * (fabs(d) + fabs(dn))) >> l << l;
+      const int mm = __ffsll((long long)small) - 1;
       if (mm == l) break;
       if (++iter > 60) {
         ok = false;
         break;
       }
-      double g = (d[l + 1] - d[l]) / (2.0 * e[l]);
-      double r = hypot(g, 1.0);
-      g = d[mm] - d[l] + e[l] / (g + (g >= 0 ? r : -r));
+      const double dl = lane_value(d, l), el = lane_value(e, l);
+      double g = (lane_value(d, l + 1) - dl) / (2.0 * el);
+      double r = hypot(g, 1.0);   // g may be huge here
+      g = lane_value(d, mm) - dl + el / (g + (g >= 0 ? r : -r));
       double s = 1.0, c = 1.0, p = 0.0;
       bool underflow = false;
       for (int i = mm - 1; i >= l; --i) {
-        double f = s * e[i];
-        const double bb = c * e[i];
-        r = hypot(f, g);
-        __syncthreads();
-        if (lane == 0) e[i + 1] = r;
+        const double ei = lane_value(e, i), di = lane_value(d, i), di1 = lane_value(d, i + 1);
+        const double f = s * ei, bb = c * ei;
+        const double r2 = f * f + g * g, ri = rsqrt_(r2);
+        r = r2 * ri;
+        if (!(r2 > 1e-290)) r = 0.0;   // both below 1e-145 of |T|
+        if (lane == i + 1) e = r;
         if (r == 0.0) {
-          if (lane == 0) {
-            d[i + 1] -= p;
-            e[mm] = 0.0;
-          }
-          __syncthreads();
+          if (lane == i + 1) d -= p;
+          if (lane == mm) e = 0.0;
           underflow = true;
           break;
         }
-        s = f / r;
-        c = g / r;
-        g = d[i + 1] - p;
-        r = (d[i] - g) * s + 2.0 * c * bb;
+        s = f * ri;
+        c = g * ri;
+        g = di1 - p;
+        r = (di - g) * s + 2.0 * c * bb;
         p = s * r;
-        __syncthreads();
-        if (lane == 0) d[i + 1] = g + p;
+        if (lane == i + 1) d = g + p;
         g = c * r - bb;
         if (lane < n) {
           const double zf = z[lane * n + i + 1], zi = z[lane * n + i];
           z[lane * n + i + 1] = s * zi + c * zf;
           z[lane * n + i] = c * zi - s * zf;
         }
-        __syncthreads();
       }
       if (underflow) continue;
-      __syncthreads();
-      if (lane == 0) {
-        d[l] -= p;
-        e[l] = g;
-        e[mm] = 0.0;
+      if (lane == l) {
+        d -= p;
+        e = g;
       }
-      __syncthreads();
+      if (lane == mm) e = 0.0;
     }
   }
   if (!ok) {   // not converged: stop the solve and report it through iters = -1
@@ -237,16 +287,21 @@ __global__ __launch_bounds__(64) void lz_expmv_check_kernel(const double *__rest
     return;
   }
   // ascending order, ties by index (a stable sort)
+  dsh[lane] = d;
+  __syncthreads();
   if (lane < n) {
     int rank = 0;
-    const double dj = d[lane];
-    for (int i = 0; i < n; ++i) rank += (d[i] < dj || (d[i] == dj && i < lane)) ? 1 : 0;
+    const double dj = d;
+    for (int i = 0; i < n; ++i) {
+      const double di = dsh[i];
+      rank += (di < dj || (di == dj && i < lane)) ? 1 : 0;
+    }
     perm[rank] = lane;
   }
   __syncthreads();
   if (lane < n) {
     const int jo = perm[lane];
-    const double ph = -tau * d[jo];
+    const double ph = -tau * ldexp(dsh[jo], ex);
     tr[lane] = cos(ph) * z[jo];   // z[0 * n + jo]
     ti[lane] = sin(ph) * z[jo];
   }
@@ -410,17 +465,17 @@ void lz_reset(hipStream_t st, LzCtl *ctl) {
   QLG_HIP(hipGetLastError());
 }
 
-void lz_gs_check(hipStream_t st, const double *ab, LzCtl *ctl, int m, int64_t dim, int64_t maxit, double err) {
+void lz_gs_check(hipStream_t st, double *ab, PartialNorm norm, LzCtl *ctl, int m, int64_t dim, int64_t maxit,
+                 double err) {
   QLG_CHECK(m + 1 <= kMaxGsDim, "device Lanczos: Krylov dimension beyond the device tridiagonal solver");
-  hipLaunchKernelGGL(lz_gs_check_kernel, dim3(1), dim3(64), 0, st, ab, ctl, m, dim, maxit, err);
+  hipLaunchKernelGGL(lz_gs_check_kernel, dim3(1), dim3(64), 0, st, ab, norm, ctl, m, dim, maxit, err);
   QLG_HIP(hipGetLastError());
 }
 
-void lz_expmv_check(hipStream_t st, const double *ab, LzCtl *ctl, double *coef_cur, double *coef_prev, double *z,
+void lz_expmv_check(hipStream_t st, double *ab, PartialNorm norm, LzCtl *ctl, double *coef_cur, double *coef_prev,
                     int m, int64_t dim, int64_t maxit, double err, double tau) {
-  (void)z;
   QLG_CHECK(m + 1 <= kZ, "device expmv: Krylov dimension beyond the device exponential");
-  hipLaunchKernelGGL(lz_expmv_check_kernel, dim3(1), dim3(64), 0, st, ab, ctl, coef_cur, coef_prev, m, dim, maxit,
+  hipLaunchKernelGGL(lz_expmv_check_kernel, dim3(1), dim3(64), 0, st, ab, norm, ctl, coef_cur, coef_prev, m, dim, maxit,
                      err, tau);
   QLG_HIP(hipGetLastError());
 }

@@ -24,6 +24,16 @@ void vec_lincomb(Ctx &c, int dtype, int64_t n, int k, const double *dev_coefs, c
                  bool complex_coefs, double br, double bi, bool use_beta, double *y);
 void vec_lanczos_residual(Ctx &c, int dtype, int64_t n, double *w, const double *v1, const double *a_dev,
                           const double *v0, const double *b_dev, double *dev_norm_out, const int *skip = nullptr);
+// One Lanczos step's vector work in two launches: a = <w, v1> (written to
+// a_out, two doubles for complex data), w <- w - a v1 - b v0, and the partial
+// sums of |w|^2, which the caller's next kernel adds up in the order of
+// reduce_partials_kernel (partial_norm).  v0 may be null.
+struct PartialNorm {
+  const double *part = nullptr;
+  int count = 0;
+};
+PartialNorm vec_lanczos_step(Ctx &c, int dtype, int64_t n, double *w, const double *v1, double *a_out,
+                             const double *v0, const double *b_dev, const int *skip);
 
 // Segmented (batched-chain) forms, real data.  A SegTable lives in device
 // memory: chunks[nchunks] of at most kSegChunk elements, each inside one

@@ -191,6 +191,48 @@ __global__ __launch_bounds__(VT) void lanczos_residual_kernel(int64_t nd, double
   if (threadIdx.x == 0) partials[blockIdx.x] = acc[0];
 }
 
+// The same update with a's partial sums added up here, by every workgroup for
+// itself and in the order of reduce_partials_kernel: the 8 KB of partials come
+// from L2, and the launch that reduced them (4.6 us, mostly latency) goes.
+template <int NC>
+__global__ __launch_bounds__(VT) void lanczos_step_kernel(int64_t nd, double *__restrict__ w,
+                                                          const double *__restrict__ v1,
+                                                          const double *__restrict__ apart, int ga,
+                                                          double *__restrict__ a_out, const double *__restrict__ v0,
+                                                          const double *__restrict__ b_ptr,
+                                                          double *__restrict__ partials,
+                                                          const int *__restrict__ skip) {
+  if (skip && *skip) return;
+  __shared__ double sh[NC][VT / 64];
+  __shared__ double a_sh;
+  double sum[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) sum[c] = 0.0;
+  for (int i = threadIdx.x; i < ga; i += VT)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) sum[c] += apart[(int64_t)i * NC + c];
+  block_sum<NC>(sum, sh);
+  if (threadIdx.x == 0) {
+    a_sh = sum[0];
+    if (blockIdx.x == 0)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) a_out[c] = sum[c];
+  }
+  __syncthreads();
+  const double a = a_sh;
+  const double b = v0 ? *b_ptr : 0.0;
+  double acc[1] = {0.0};
+  const int64_t stride = (int64_t)gridDim.x * VT;
+  for (int64_t i = (int64_t)blockIdx.x * VT + threadIdx.x; i < nd; i += stride) {
+    double g = w[i] - a * v1[i];
+    if (v0) g -= b * v0[i];
+    w[i] = g;
+    acc[0] += g * g;
+  }
+  block_sum<1>(acc, sh);
+  if (threadIdx.x == 0) partials[blockIdx.x] = acc[0];
+}
+
 // ---------------------------------------------------------------------------
 static int grid_for(int64_t n) {
   int64_t g = (n + 4 * VT - 1) / (4 * VT);
@@ -277,6 +319,25 @@ void vec_lanczos_residual(Ctx &c, int dtype, int64_t n, double *w, const double 
                      skip);
   hipLaunchKernelGGL(reduce_partials_kernel<1>, dim3(1), dim3(VT), 0, c.stream, part, g, dev_norm_out, 1, skip);
   QLG_HIP(hipGetLastError());
+}
+
+PartialNorm vec_lanczos_step(Ctx &c, int dtype, int64_t n, double *w, const double *v1, double *a_out,
+                             const double *v0, const double *b_dev, const int *skip) {
+  const bool cplx = dtype == QLG_C128;
+  const int64_t nd = n * elem_doubles(dtype);
+  const int ga = grid_for(n), g = grid_for(nd);
+  double *apart = c.partials.as<double>(), *part = apart + 2 * kMaxPartials;
+  if (cplx) {
+    hipLaunchKernelGGL(dot_partial_kernel<true>, dim3(ga), dim3(VT), 0, c.stream, n, w, v1, apart, skip);
+    hipLaunchKernelGGL(lanczos_step_kernel<2>, dim3(g), dim3(VT), 0, c.stream, nd, w, v1, apart, ga, a_out, v0, b_dev,
+                       part, skip);
+  } else {
+    hipLaunchKernelGGL(dot_partial_kernel<false>, dim3(ga), dim3(VT), 0, c.stream, n, w, v1, apart, skip);
+    hipLaunchKernelGGL(lanczos_step_kernel<1>, dim3(g), dim3(VT), 0, c.stream, nd, w, v1, apart, ga, a_out, v0, b_dev,
+                       part, skip);
+  }
+  QLG_HIP(hipGetLastError());
+  return PartialNorm{part, g};
 }
 
 // ---------------------------------------------------------------------------
