@@ -34,7 +34,7 @@ constexpr int PAD = 1;
 }
 
 template <int BM, int BN, int BK, bool CPLX>
-__global__ __launch_bounds__(256) void grouped_gemm_f64_kernel(const GemmTile *__restrict__ tiles,
+__global__ __launch_bounds__(256, BM * BN * (CPLX ? 2 : 1) >= 128 * 128 ? 1 : 2) void grouped_gemm_f64_kernel(const GemmTile *__restrict__ tiles,
                                                                const GemmTask *__restrict__ tasks,
                                                                const GemmSeg *__restrict__ segs,
                                                                Slots slots, int ntiles) {

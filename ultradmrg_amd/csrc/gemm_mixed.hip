@@ -95,7 +95,7 @@ __device__ inline void store_tile(const GemmTask &tk, const GemmTile &tl, const 
 // ---------------------------------------------------------------------------
 // FP32 MFMA.  LDS: As[k][m], Bs[k][n] (FP32), BK-deep slices, ping-pong.
 template <int BM, int BN, int BK, typename TB, typename TC>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const GemmTile *__restrict__ tiles,
+__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmTile *__restrict__ tiles,
                                                        const GemmTask *__restrict__ tasks,
                                                        const GemmSeg *__restrict__ segs, Slots slots, int ntiles) {
   constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16;
@@ -257,7 +257,7 @@ __device__ inline void split8(const float (&x)[8], bf16x8 (&p)[NPIECE]) {
 // tile's prologue and epilogue) and for the 3-term mode (two pieces: less
 // split work to save).
 template <int BM, int BN, int NPC, typename TB, typename TC>
-__global__ __launch_bounds__(256) void gemm_bf16_frag_kernel(const GemmTile *__restrict__ tiles,
+__global__ __launch_bounds__(256, 2) void gemm_bf16_frag_kernel(const GemmTile *__restrict__ tiles,
                                                         const GemmTask *__restrict__ tasks,
                                                         const GemmSeg *__restrict__ segs, Slots slots, int ntiles) {
   constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16;
@@ -449,7 +449,7 @@ __device__ inline void split4(const float (&x)[4], bf16x4 (&p)[NPIECE]) {
 }  // namespace
 
 template <int BM, int BN, int NPC, typename TB, typename TC>
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(const GemmTile *__restrict__ tiles,
+__global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(const GemmTile *__restrict__ tiles,
                                                         const GemmTask *__restrict__ tasks,
                                                         const GemmSeg *__restrict__ segs, Slots slots, int ntiles) {
   constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16;
@@ -643,7 +643,7 @@ __device__ inline float2 load_cplx_as_f32(__amdgpu_buffer_rsrc_t r, uint32_t ele
 }
 
 template <int BM, int BN, int NPC, typename TB, typename TC>
-__global__ __launch_bounds__(256) void gemm_bf16_cplx_kernel(const GemmTile *__restrict__ tiles,
+__global__ __launch_bounds__(256, 2) void gemm_bf16_cplx_kernel(const GemmTile *__restrict__ tiles,
                                                              const GemmTask *__restrict__ tasks,
                                                              const GemmSeg *__restrict__ segs, Slots slots,
                                                              int ntiles) {
@@ -832,7 +832,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_cplx_kernel(const GemmTile *__r
 constexpr int kSliceBufs = 1;
 
 template <int BM, int BN, int NPC, typename TB, typename TC, bool BPLANAR>
-__global__ __launch_bounds__(256) void gemm_bf16p_kernel(const GemmTile *__restrict__ tiles,
+__global__ __launch_bounds__(256, 2) void gemm_bf16p_kernel(const GemmTile *__restrict__ tiles,
                                                          const GemmTask *__restrict__ tasks,
                                                          const GemmSeg *__restrict__ segs, Slots slots, int ntiles) {
   constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16;

@@ -64,7 +64,7 @@ struct Mfma<float> {    // v_mfma_f32_16x16x4: D lane l, reg r -> row 4 (l / 16)
 // FP32 result x, h = bf16(x), m = bf16(x - h), l = bf16(x - h - m), plane q
 // at yps elements after plane q - 1 (the operand of the pre-split stage 3).
 template <int BM, int BN, bool CPLX, typename T, int OUTP = 0>
-__global__ __launch_bounds__(256) void mpo_stage_kernel(const ChanTile *__restrict__ tiles,
+__global__ __launch_bounds__(256, 2) void mpo_stage_kernel(const ChanTile *__restrict__ tiles,
                                                         const RowDesc *__restrict__ rows, const T *__restrict__ C,
                                                         const T *__restrict__ X, T *__restrict__ Y,
                                                         const int *__restrict__ skip, int64_t yps, int ntiles) {
