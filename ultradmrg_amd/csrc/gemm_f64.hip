@@ -428,9 +428,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK, FM * FN * (CPLX ? 2 : 1) <= 8 ? 
       // leaves the later slices' loads in flight
       __builtin_amdgcn_sched_barrier(0);
     };
-    auto multiply = [&](int d) {
+    // a slice's MFMAs; its k-steps from `left` on are past K (the last slice of
+    // a short K is a good part of it)
+    auto multiply = [&](int d, int left) {
 #pragma unroll
-      for (int t = 0; t < KD / 4; ++t)
+      for (int t = 0; t < KD / 4; ++t) {
+        if (4 * t >= left) break;
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -443,7 +446,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK, FM * FN * (CPLX ? 2 : 1) <= 8 ? 
               acc[1][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[1], b[0], acc[1][i][j], 0, 0, 0);
             }
           }
+      }
     };
+    auto left = [&](int n) { return K - (n * WK + wk) * KD; };
 #pragma unroll
     for (int d = 0; d < kDepth; ++d) fetch(d, d);
     int n = 0;
@@ -452,17 +457,17 @@ __global__ __launch_bounds__(64 * WM * WN * WK, FM * FN * (CPLX ? 2 : 1) <= 8 ? 
     for (; n + 2 * kDepth <= ns; n += kDepth)
 #pragma unroll
       for (int d = 0; d < kDepth; ++d) {
-        multiply(d);
+        multiply(d, KD);
         fetch(d, n + d + kDepth);
       }
 #pragma unroll
     for (int d = 0; d < kDepth; ++d) {
-      if (n + d < ns) multiply(d);
+      if (n + d < ns) multiply(d, left(n + d));
       if (n + d + kDepth < ns) fetch(d, n + d + kDepth);
     }
 #pragma unroll
     for (int d = 0; d < kDepth - 1; ++d)
-      if (n + d + kDepth < ns) multiply(d);
+      if (n + d + kDepth < ns) multiply(d, left(n + d + kDepth));
   }
 
   // output row addresses: a row-address table or a plain row stride
