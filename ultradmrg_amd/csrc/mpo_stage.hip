@@ -63,6 +63,9 @@ struct Mfma<float> {    // v_mfma_f32_16x16x4: D lane l, reg r -> row 4 (l / 16)
 // OUTP > 0 (real FP32 only): Y is written as OUTP bf16 piece planes of each
 // FP32 result x, h = bf16(x), m = bf16(x - h), l = bf16(x - h - m), plane q
 // at yps elements after plane q - 1 (the operand of the pre-split stage 3).
+// There a lane holds two neighbouring positions (blocks j, j + 1 interleaved),
+// so that a plane is written in 4-byte pieces: with 2-byte ones the stage was
+// bound by its stores (a converged D=2000 profile: PLACEHOLDER).
 template <int BM, int BN, bool CPLX, typename T, int OUTP = 0>
 __global__ __launch_bounds__(256, 2) void mpo_stage_kernel(const ChanTile *__restrict__ tiles,
                                                         const RowDesc *__restrict__ rows, const T *__restrict__ C,
@@ -112,12 +115,13 @@ __global__ __launch_bounds__(256, 2) void mpo_stage_kernel(const ChanTile *__res
     rout[tid] = dout;
   }
 
+  constexpr bool PAIR = OUTP > 0 && FN % 2 == 0;   // interleaved blocks
   // this lane's columns: (a', b) positions of its B fragments
   int apj[FN], bj[FN];
   bool okj[FN];
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
-    const int col = tl.n0 + wave * WN + j * 16 + (lane & 15);
+    const int col = tl.n0 + wave * WN + (PAIR ? (j / 2) * 32 + 2 * (lane & 15) + (j & 1) : j * 16 + (lane & 15));
     okj[j] = col < N;
     apj[j] = okj[j] ? col / tk.Db : 0;
     bj[j] = okj[j] ? col % tk.Db : 0;
@@ -233,6 +237,38 @@ __global__ __launch_bounds__(256, 2) void mpo_stage_kernel(const ChanTile *__res
       ro[i][r] = d.off;
       rr[i][r] = (int32_t)d.rs;
     }
+  if constexpr (PAIR) {
+    typedef unsigned int u32u __attribute__((aligned(2)));
+    __bf16 *P = reinterpret_cast<__bf16 *>(Y);
+#pragma unroll
+    for (int j = 0; j < FN; j += 2) {
+      if (!okj[j]) continue;
+      const bool both = okj[j + 1], run = both && apj[j + 1] == apj[j];   // positions of one run are neighbours
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (tl.m0 + i * 16 + MF::row(lane, r) >= M) continue;
+          const int64_t i0 = ro[i][r] + (int64_t)apj[j] * rr[i][r] + bj[j];
+          const int64_t i1 = ro[i][r] + (int64_t)apj[j + 1] * rr[i][r] + bj[j + 1];
+          float x = acc[0][i][j][r], y = acc[0][i][j + 1][r];
+#pragma unroll
+          for (int q = 0; q < OUTP; ++q) {
+            const __bf16 hx = (__bf16)x, hy = (__bf16)y;
+            x -= (float)hx;
+            y -= (float)hy;
+            if (run) {
+              *reinterpret_cast<u32u *>(P + q * yps + i0) =
+                  (unsigned)__builtin_bit_cast(unsigned short, hx) | (unsigned)__builtin_bit_cast(unsigned short, hy) << 16;
+            } else {
+              P[q * yps + i0] = hx;
+              if (both) P[q * yps + i1] = hy;
+            }
+          }
+        }
+    }
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
     if (!okj[j]) continue;
