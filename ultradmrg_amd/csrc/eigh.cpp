@@ -151,7 +151,7 @@ static void solve_group(rocblas_handle h, int dtype, const qlg_eigh_group &g, do
     throw Error(QLG_ERR_HIP, "rocSOLVER syevd/heevd returned status " + std::to_string((int)st));
 }
 
-void eigh_batched(Ctx &c, int dtype, int64_t ngroups, const qlg_eigh_group *groups) {
+void eigh_batched(Ctx &c, int dtype, int64_t ngroups, const qlg_eigh_group *groups, bool use_small) {
   QLG_CHECK(dtype == QLG_F64 || dtype == QLG_C128, "eigh: dtype must be F64 or C128");
   QLG_CHECK(ngroups >= 0 && (ngroups == 0 || groups), "eigh: bad group list");
   if (ngroups == 0) return;
@@ -182,7 +182,7 @@ void eigh_batched(Ctx &c, int dtype, int64_t ngroups, const qlg_eigh_group *grou
   // latency per column) with a mild batch term
   std::vector<int64_t> order, small;
   for (int64_t k = 0; k < ngroups; ++k)
-    (dtype == QLG_F64 && groups[k].n <= kSmallEigh ? small : order).push_back(k);
+    (use_small && dtype == QLG_F64 && groups[k].n <= kSmallEigh ? small : order).push_back(k);
   if (!order.empty()) make_lanes(p);
   auto cost = [&](int64_t k) { return (double)groups[k].n * (1.0 + 0.05 * (double)groups[k].batch); };
   std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return cost(a) > cost(b); });

@@ -65,13 +65,13 @@ struct Bucket {
   int64_t xbase = 0, gbase = 0, rbase = 0;
 };
 
-// Orders up to kSmallEigh are solved in LDS, a real bucket per launch, and gain from
-// buckets of their own; a complex one is a divide-and-conquer call whose time
-// is its largest order's, so small complex sectors share the first large one.
-int64_t bucket_bound(int64_t n, bool cplx) {
-  if (!cplx)
-    for (int64_t b : {int64_t(1), int64_t(16), int64_t(32), int64_t(48), int64_t(kSmallEigh)})
-      if (n <= b) return b;
+// `small`: the call's sectors are all real and of at most kSmallSector rows, and
+// are solved in LDS (eigh_small.hip), where a bucket costs its own order.
+// Otherwise a bucket is a divide-and-conquer call whose time is its largest
+// order's, so the smaller sectors share the first one.
+constexpr int64_t kSmallSector = 28;
+int64_t bucket_bound(int64_t n, bool small) {
+  if (small) return n <= 1 ? 1 : n <= 16 ? 16 : 32;
   static const int64_t bounds[] = {1, 256, 512, 768, 1024, 1536, 2048, 3072, 4096, 6144, 8192};
   for (int64_t b : bounds)
     if (n <= b) return b;
@@ -246,7 +246,9 @@ SvdResult *block_svd(Ctx &c, const qlg_bsten *desc, int ldims, const int32_t *ld
   }
   // ---- buckets ------------------------------------------------------------------------
   std::map<int64_t, std::vector<int>> raw;
-  for (int s : order) raw[bucket_bound(sec[s].n, cplx)].push_back(s);
+  bool small = !cplx;
+  for (const Sector &s : sec) small = small && s.n <= kSmallSector;
+  for (int s : order) raw[bucket_bound(sec[s].n, small)].push_back(s);
   std::vector<Bucket> bk;
   int64_t xtot = 0, gtot = 0, rtot = 0, nsv = 0;
   for (auto &kv : raw) {
@@ -402,7 +404,7 @@ SvdResult *block_svd(Ctx &c, const qlg_bsten *desc, int ldims, const int32_t *ld
         groups.push_back(qlg_eigh_group{B.b, (int64_t)B.secs.size(), G.as<double>() + B.gbase * ed,
                                         W.as<double>() + wbase[i]});
       }
-      eigh_batched(c, t.dtype, (int64_t)groups.size(), groups.data());
+      eigh_batched(c, t.dtype, (int64_t)groups.size(), groups.data(), small);
       if (!cplx) break;
       // undo the rotation on the rows of E^H: r <- r H2, then r <- r H1
       size_t pos = 0;
@@ -673,7 +675,7 @@ SvdResult *block_svd(Ctx &c, const qlg_bsten *desc, int ldims, const int32_t *ld
             groups.push_back(qlg_eigh_group{kv.first, (int64_t)kv.second.size(), Gs.as<double>() + q0.gs,
                                             Ws.as<double>() + q0.ws});
           }
-          eigh_batched(c, QLG_F64, (int64_t)groups.size(), groups.data());
+          eigh_batched(c, QLG_F64, (int64_t)groups.size(), groups.data(), small);
           {
             // rows of the eigenvector buffer kb - k .. kb - 1: the valid (ascending) eigenvectors
             GemmBatch gb(c, false);
