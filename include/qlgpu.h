@@ -337,8 +337,8 @@ int qlg_svd_destroy(qlg_svd r);
  * for callers with their own batches.  Group k holds batch matrices of order n, row-major and
  * Hermitian, at a (dtype QLG_F64 or QLG_C128); on return row j of each matrix
  * holds eigenvector j (complex-conjugated for QLG_C128) and w[0..n) its
- * eigenvalues in ascending order.  Divide and conquer; groups run
- * concurrently.  The call returns after the work is complete (it checks the
+ * eigenvalues in ascending order.  Real groups of order 32 and less: cyclic
+ * Jacobi in LDS; all others: divide and conquer.  Groups run concurrently.  The call returns after the work is complete (it checks the
  * solver's convergence flags); QLG_ERR_NUMERIC if a matrix did not converge. */
 typedef struct {
   int64_t n;      /* order of each matrix   */

@@ -8,6 +8,8 @@
 // bound by host-side launch latency, not by the device.  Groups are therefore
 // spread over kLanes lanes, each a host thread with its own stream and rocBLAS
 // handle, forked from and joined back into the context stream with events.
+// Real groups of order kSmallEigh and less run in LDS instead (eigh_small.hip),
+// on the context stream beside the lanes, where the caller allows it.
 //
 // Initialisation is serial.  rocBLAS loads its Tensile kernel libraries
 // lazily, on a handle's first GEMM; four lanes making their first call at the

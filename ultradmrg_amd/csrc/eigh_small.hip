@@ -7,9 +7,10 @@
 // spends several launches per column on them (0.6 ms of kernels and over 1 ms
 // of host time at order 32, whatever the batch); here a whole batch is one
 // launch.  A sweep of a 20-site chain at D = 48, whose 36 updates are mostly
-// such decompositions, went from 156 to 100 ms.  A round is bound by latency: the rotation angles (two reciprocals
-// and two reciprocal square roots in sequence), two barriers and the LDS round
-// trips between them; a matrix takes n - 1 rounds a sweep and 6 to 9 sweeps.
+// such decompositions, went from 156 to 100 ms.  A round is bound by latency:
+// the rotation angles (two reciprocals and two reciprocal square roots in
+// sequence), two barriers and the LDS round trips between them; a matrix takes
+// n - 1 rounds a sweep and 6 to 9 sweeps.
 //
 // A pair is rotated while |a_pq| > 4 eps sqrt(|a_pp a_qq|) and above 1e-3 eps
 // |A|_F: the Gram matrices' small eigenvalues keep their relative accuracy as

@@ -1,16 +1,20 @@
-// Grouped FP64 GEMM on CDNA4 MFMA (v_mfma_f64_16x16x4_f64).
+// Grouped FP64 GEMM on CDNA4 MFMA (v_mfma_f64_16x16x4_f64), in two kernels:
+// direct_gemm_f64_kernel (further down) for the matvec's two contractions,
+// whose operands the planner lays out for it, and grouped_gemm_f64_kernel for
+// operands in any order (environment updates, contractions, the SVD's
+// products) and for matvec plans whose spans the direct kernel cannot address.
 //
-// One workgroup (4 wavefronts, 2x2) computes one BM x BN output tile of one
-// task and walks the task's K-segments in order.  BK-deep slices of A and B
-// are staged through two LDS buffers (ping-pong): the raw buffer loads of
-// slice i+1 are issued before the MFMAs of slice i and land in registers,
-// which are written to the other LDS buffer afterwards, so each K step costs
-// one barrier and the load latency hides behind the MFMA work.  Operands are
-// read with raw buffer loads whose out-of-range elements come back as zero
-// (tile_io.h), so the loads carry no branch and no select.  Slices run as
-// straight-line code, which lets the LDS fragment reads of one 4-deep
-// sub-step overlap the MFMAs of the previous one (a segment's last slice is
-// zero-filled past K and runs the same code).  Each wave owns a
+// grouped_gemm_f64_kernel: one workgroup (4 wavefronts, 2x2) computes one BM x
+// BN output tile of one task and walks the task's K-segments in order.
+// BK-deep slices of A and B are staged through two LDS buffers (ping-pong): the
+// raw buffer loads of slice i+1 are issued before the MFMAs of slice i and
+// land in registers, which are written to the other LDS buffer afterwards, so
+// each K step costs one barrier and the load latency hides behind the MFMA
+// work.  Operands are read with raw buffer loads whose out-of-range elements
+// come back as zero (tile_io.h), so the loads carry no branch and no select.
+// Slices run as straight-line code, which lets the LDS fragment reads of one
+// 4-deep sub-step overlap the MFMAs of the previous one (a segment's last
+// slice is zero-filled past K and runs the same code).  Each wave owns a
 // (BM/2) x (BN/2) sub-tile of 16x16 MFMA blocks; thin tiles (BN = 16, for
 // tasks with few columns) stack the four waves along M.
 //
@@ -318,6 +322,13 @@ static void launch_shape(int bm, int bn, int bk, const GemmTile *tiles, const Ge
 // slices w, w + WK, ...; the parts are summed through LDS in order at the end.
 // Small tiles use WK > 1, so that long-K tasks with few columns keep every
 // SIMD busy.
+//
+// Measured per launch, LDS kernel -> this one (kernel trace): Hubbard D=2000
+// (5.6 GFLOP each) stage 1 177 -> 145 us, stage 3 188 (and 17 for split-K's
+// reduce) -> 137 us; dense 8 x (4096 x 4096 x 2048) 72 TFLOP/s.  The two-waves
+// launch bound keeps the accumulators in vector registers: without it each
+// slice moved them to and from the accumulation registers.  What is left is
+// padding to 16-wide blocks, the last wave of tiles and the stores of T1.
 // ---------------------------------------------------------------------------
 __device__ inline double2 load_pair(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   typedef double d2 __attribute__((ext_vector_type(2)));

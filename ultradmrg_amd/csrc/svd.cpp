@@ -9,7 +9,7 @@
 // first (transposed when it has more rows than columns), into padded batches
 // of a few size buckets, scaled to unit Frobenius norm, and decomposed
 // through its Gram matrix X X^H (grouped FP64 GEMM, rocSOLVER divide and
-// conquer on four lanes, eigh.cpp):
+// conquer on four lanes, eigh.cpp, or in LDS when every sector is small):
 //   X = E S P,  rows of R = E^H X are s_j p_j,  s_j = |R_j|
 // (the back-projected row norm has absolute error ~eps s_max, where
 // sqrt(lambda_j) would have eps s_max^2 / s_j).  Eigenvectors of tiny
