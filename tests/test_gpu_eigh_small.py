@@ -76,3 +76,23 @@ def test_mixed_groups():
                 continue
             n = a.shape[0]
             assert np.linalg.norm(a @ vi - vi * wi, 2) <= 4 * n * EPS * np.linalg.norm(a, 2)
+
+
+@pytest.mark.parametrize("power", [-1030, -665, 665, 1010])
+@pytest.mark.parametrize("n", [2, 17, 32])
+def test_any_scale(n, power):
+    """Matrices scaled by 2^power, down to denormal elements and up to where their
+    squares overflow.  The bars are those of the unscaled matrix (the input's own
+    rounding to denormal numbers is part of the matrix) plus the rounding of a
+    value to a denormal number, 2^-1075."""
+    print(f"[case] order {n} scaled by 2^{power}", flush=True)
+    rng = np.random.default_rng(n)
+    mats = np.stack([(lambda a: np.ldexp((a + a.T) / 2, power))(_matrix(k, n, rng)) for k in KINDS])
+    (w, v), = eigh_batched([torch.from_numpy(mats.copy()).cuda()])
+    w, v = np.ldexp(w.cpu().numpy(), -power), v.cpu().numpy()
+    for k, a, wi, vi in zip(KINDS, np.ldexp(mats, -power), w, v):
+        bar = 4 * n * EPS * max(np.linalg.norm(a, 2), np.finfo(float).tiny) + 2.0 ** max(-1075 - power, -1000)
+        assert np.all(np.diff(wi) >= 0), k
+        assert np.abs(wi - np.linalg.eigvalsh(a)).max() <= bar, k
+        assert np.linalg.norm(a @ vi - vi * wi, 2) <= bar, k
+        assert np.linalg.norm(vi.T @ vi - np.eye(n), 2) <= 8 * n * EPS, k

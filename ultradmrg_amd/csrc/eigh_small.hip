@@ -19,6 +19,9 @@
 // off-diagonal elements are within 16 eps |A|_F.
 #include <hip/hip_runtime.h>
 
+#include <cfloat>
+#include <cmath>
+
 #include "common.h"
 #include "eigh.h"
 
@@ -41,15 +44,22 @@ __device__ inline double rsqrt_(double x) {
   return fma(0.5 * r, fma(-x * r, r, 1.0), r);
 }
 
-__device__ inline double block_sum(double v, double *red) {
+template <class Op>
+__device__ inline double block_reduce(double v, double *red, Op op) {
   const int tid = threadIdx.x;
-  for (int o = 32; o; o >>= 1) v += __shfl_xor(v, o);
+  for (int o = 32; o; o >>= 1) v = op(v, __shfl_xor(v, o));
   __syncthreads();
   if ((tid & 63) == 0) red[tid >> 6] = v;
   __syncthreads();
-  double s = 0.0;
-  for (int i = 0; i < (int)blockDim.x / 64; ++i) s += red[i];
-  return s;
+  v = red[0];
+  for (int i = 1; i < (int)blockDim.x / 64; ++i) v = op(v, red[i]);
+  return v;
+}
+__device__ inline double block_sum(double v, double *red) {
+  return block_reduce(v, red, [](double x, double y) { return x + y; });
+}
+__device__ inline double block_max(double v, double *red) {
+  return block_reduce(v, red, [](double x, double y) { return fmax(x, y); });
 }
 }  // namespace
 
@@ -66,31 +76,33 @@ __global__ __launch_bounds__(1024) void jacobi_eigh_kernel(double *__restrict__ 
   double *A = lds, *V = lds + n * ld;
   double *ga = a + (int64_t)blockIdx.x * n * n;
   double *gw = w + (int64_t)blockIdx.x * n;
-  double fro = 0.0;
+  double big = 0.0;   // largest magnitude; infinite if any element is not finite
   for (int e = tid; e < n * n; e += nt) {
     const int i = e / n, j = e % n;
     // the lower triangle is the input, as for the library's solver
     const double v = ga[i >= j ? e : j * n + i];
     A[i * ld + j] = v;
     V[i * ld + j] = i == j ? 1.0 : 0.0;
-    fro += v * v;
+    big = fmax(big, fabs(v) <= DBL_MAX ? fabs(v) : HUGE_VAL);
   }
-  fro = sqrt(block_sum(fro, red));
-  if (!(fro < 1.0e300)) {   // NaN or infinity in the input: NaN out
-    for (int e = tid; e < n * n; e += nt) ga[e] = fro - fro;
-    for (int i = tid; i < n; i += nt) gw[i] = fro - fro;
+  big = block_max(big, red);
+  if (big > DBL_MAX) {   // NaN or infinity in the input: NaN out
+    for (int e = tid; e < n * n; e += nt) ga[e] = big - big;
+    for (int i = tid; i < n; i += nt) gw[i] = big - big;
     if (tid == 0) info[blockIdx.x] = 0;
     return;
   }
-  // scaled by a power of two to a norm in [1, 2): no product below overflows,
-  // and no reciprocal meets a denormal number
-  int ex = 0;
-  if (fro > 0.0) {
-    ex = ilogb(fro);
-    fro = ldexp(fro, -ex);
-    for (int e = tid; e < n * n; e += nt) A[e / n * ld + e % n] = ldexp(A[e / n * ld + e % n], -ex);
-    __syncthreads();
+  // scaled by a power of two to a largest element in [1, 2), whatever the
+  // input's range: no product below overflows, and no reciprocal meets a
+  // denormal number
+  const int ex = big > 0.0 ? ilogb(big) : 0;
+  double fro = 0.0;
+  for (int e = tid; e < n * n; e += nt) {   // (the thread's own elements)
+    double &v = A[e / n * ld + e % n];
+    v = ldexp(v, -ex);
+    fro += v * v;
   }
+  fro = sqrt(block_sum(fro, red));
   const int np = (n + 1) & ~1, half = np / 2;   // odd n: one index sits out each round
   const int lgh = half > 1 ? 32 - __clz(half - 1) : 0, lgn = n > 1 ? 32 - __clz(n - 1) : 0;
   const double floor_abs = 1e-3 * kEps * fro;
