@@ -334,12 +334,14 @@ int qlg_svd_destroy(qlg_svd r);
 
 /* ---- batched Hermitian eigen-decomposition ---------------------------------------
  * The solver qlg_block_svd runs on the Gram matrices of its sectors, exported
- * for callers with their own batches.  Group k holds batch matrices of order n, row-major and
- * Hermitian, at a (dtype QLG_F64 or QLG_C128); on return row j of each matrix
+ * for callers with their own batches.  Group k holds batch matrices of order n,
+ * row-major and Hermitian, at a (dtype QLG_F64 or QLG_C128), of which the
+ * diagonal and the upper triangle are read; on return row j of each matrix
  * holds eigenvector j (complex-conjugated for QLG_C128) and w[0..n) its
  * eigenvalues in ascending order.  Real groups of order 32 and less: cyclic
- * Jacobi in LDS; all others: divide and conquer.  Groups run concurrently.  The call returns after the work is complete (it checks the
- * solver's convergence flags); QLG_ERR_NUMERIC if a matrix did not converge. */
+ * Jacobi in LDS; all others: divide and conquer.  Groups run concurrently.  The
+ * call returns after the work is complete (it checks the solver's convergence
+ * flags); QLG_ERR_NUMERIC if a matrix did not converge. */
 typedef struct {
   int64_t n;      /* order of each matrix   */
   int64_t batch;  /* matrices in the group  */

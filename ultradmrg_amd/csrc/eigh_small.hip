@@ -79,8 +79,9 @@ __global__ __launch_bounds__(1024) void jacobi_eigh_kernel(double *__restrict__ 
   double big = 0.0;   // largest magnitude; infinite if any element is not finite
   for (int e = tid; e < n * n; e += nt) {
     const int i = e / n, j = e % n;
-    // the lower triangle is the input, as for the library's solver
-    const double v = ga[i >= j ? e : j * n + i];
+    // the row-major upper triangle is the input, as for the library's solver
+    // (which takes the lower one of the same memory read column-major)
+    const double v = ga[i <= j ? e : j * n + i];
     A[i * ld + j] = v;
     V[i * ld + j] = i == j ? 1.0 : 0.0;
     big = fmax(big, fabs(v) <= DBL_MAX ? fabs(v) : HUGE_VAL);
