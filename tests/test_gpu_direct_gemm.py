@@ -71,6 +71,19 @@ def test_edge_sectors(monkeypatch, degs, cplx, shape):
     assert _err(H @ to_device(psi), ref) < 1e-12
 
 
+@pytest.mark.parametrize("shape", ["128x64", "64x128", "128x128"])
+@pytest.mark.parametrize("degs", [EDGES, LONG], ids=["edges", "long"])
+def test_wide_complex_tiles(monkeypatch, degs, shape):
+    """Complex tiles that only the LDS-staged kernel has, pinned: it runs on the same
+    k-major operands and row tables."""
+    print(f"[case] {degs} complex {shape}", flush=True)
+    monkeypatch.setenv("QLG_TILES", f"{shape},16x128,{shape}")
+    eff, psi = _problem(degs, 5, True)
+    ref = eff_ham_mul_two_site_state(eff, psi)
+    H = EffectiveHamiltonian([to_device(t) for t in eff], to_device(psi))
+    assert _err(H @ to_device(psi), ref) < 1e-12
+
+
 @pytest.mark.parametrize("first", ["fp64", "bf16x6"])
 def test_plan_switches_layouts(first):
     """One plan through FP64, both kinds of reduced layouts and back: the FP64

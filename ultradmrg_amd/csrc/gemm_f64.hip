@@ -564,6 +564,11 @@ static void launch_direct(int bm, int bn, const GemmTile *tiles, const GemmTask 
   throw Error(QLG_ERR_UNSUPPORTED, "unsupported FP64 tile shape");
 }
 
+// Complex tiles end at 64 x 64: two accumulator planes of a 128-wide tile leave
+// no registers for fragments in flight.  A plan pinned to a wider one
+// (QLG_TILES) runs on the LDS kernel, which has it.
+bool direct_gemm_shape(int bm, int bn, bool cplx) { return !cplx || (bm <= 64 && bn >= 32 && bn <= 64); }
+
 void launch_direct_gemm_f64(int bm, int bn, bool cplx, const GemmTile *tiles, const GemmTask *tasks,
                             const GemmSeg *segs, const Slots &slots, int ntiles, hipStream_t st) {
   if (ntiles <= 0) return;

@@ -1085,7 +1085,7 @@ void Plan::launch_stage(int i, const Slots &s) {
     // stage 3: A = Y, B = R panels (transposed), C = the Krylov output (FP64, row table)
     launch_grouped_gemm_mixed(precision, g.bm, g.bn, i == 0, i == 2, cplx, g.d_tiles.as<GemmTile>(),
                               g.d_tasks.as<GemmTask>(), g.d_segs.as<GemmSeg>(), s, (int)g.tiles.size(), stream);
-  } else if (g.direct) {
+  } else if (g.direct && direct_gemm_shape(g.bm, g.bn, cplx)) {
     launch_direct_gemm_f64(g.bm, g.bn, cplx, g.d_tiles.as<GemmTile>(), g.d_tasks.as<GemmTask>(),
                            g.d_segs.as<GemmSeg>(), s, (int)g.tiles.size(), stream);
   } else {

@@ -213,7 +213,9 @@ std::string tile_signature(const Stage &s, int stage, int variant);
 
 void launch_grouped_gemm_f64(int bm, int bn, bool cplx, const GemmTile *tiles, const GemmTask *tasks,
                              const GemmSeg *segs, const Slots &slots, int ntiles, hipStream_t st);
-// fragments straight from memory (gemm_f64.hip): a stage with Stage::direct set
+// fragments straight from memory (gemm_f64.hip): a stage with Stage::direct set,
+// on the tile shapes that direct_gemm_shape names
+bool direct_gemm_shape(int bm, int bn, bool cplx);
 void launch_direct_gemm_f64(int bm, int bn, bool cplx, const GemmTile *tiles, const GemmTask *tasks,
                             const GemmSeg *segs, const Slots &slots, int ntiles, hipStream_t st);
 // sums the split-K partial panels of a stage into its outputs (FP64 / complex128)
