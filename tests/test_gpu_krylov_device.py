@@ -179,3 +179,60 @@ def test_reorthogonalisation(passes):
     got = to_oracle(rc.expmv, psi).to_dense().reshape(-1)
     assert float(np.linalg.norm(got - exact) / np.linalg.norm(exact)) < 1e-10
     Hc.close()
+
+
+def _expmv_extended(H, x, tau, k):
+    """k Lanczos steps and exp(-i tau T) e_1 in extended precision (the sum of the
+    exponential's series over 64 substeps)."""
+    LD, CLD = np.longdouble, np.clongdouble
+    nrm = np.sqrt((np.abs(x) ** 2).sum())
+    V, T = [x / nrm], np.zeros((k, k), LD)
+    for m in range(k):
+        w = H @ V[m]
+        T[m, m] = (V[m].conj() * w).sum().real
+        w = w - T[m, m] * V[m] - (T[m, m - 1] * V[m - 1] if m else 0)
+        if m + 1 < k:
+            T[m, m + 1] = T[m + 1, m] = np.sqrt((np.abs(w) ** 2).sum())
+            V.append(w / T[m, m + 1])
+    c = np.zeros(k, CLD)
+    c[0] = nrm
+    A = CLD(-1j) * LD(tau) / 64 * T
+    for _ in range(64):
+        t = c
+        for j in range(1, 40):
+            t = A @ t / LD(j)
+            c = c + t
+    return sum(v * z for v, z in zip(V, c))
+
+
+def test_expmv_rounding(monkeypatch):
+    """The device's exponential rounds no worse than the host form, whose divisions
+    and square roots are correctly rounded: the mean error over 32 states against
+    the same Krylov steps in extended precision."""
+    print("[case] expmv rounding", flush=True)
+    monkeypatch.setenv("QLG_TILES", "32x32,16x128,32x32")   # one order of sums wherever it runs
+    eff, psi = _complex_problem()
+    e = [t.to_dense().astype(np.clongdouble) for t in eff]
+    t = np.tensordot(e[0], e[1], ([1], [0]))                         # x a s t y
+    t = np.tensordot(t, e[2], ([4], [0]))                            # x a s t u v z
+    Hd = np.tensordot(t, e[3], ([6], [1])).transpose(0, 3, 5, 6, 1, 2, 4, 7)   # x t v b a s u c
+    n = int(np.prod(Hd.shape[:4]))
+    Hd = Hd.reshape(n, n)
+    tau, k = 0.05, 10
+    H = EffectiveHamiltonian([to_device(t) for t in eff], to_device(psi))
+    err = {"device": [], "host": []}
+    rng = np.random.default_rng(5)
+    for _ in range(32):
+        x = random_fill(BSTensor(psi.indexes, np.complex128), (0,), rng, complex_=True)
+        ref = _expmv_extended(Hd, x.to_dense().reshape(-1).astype(np.clongdouble), tau, k)
+        for form in err:
+            with _env(QLG_KRYLOV_HOST=int(form == "host")):
+                r = H.expmv(to_device(x), tau, LanczosParams(1e-30, k))
+            got = to_oracle(r.expmv, psi).to_dense().reshape(-1)
+            err[form].append(float(np.linalg.norm((got - ref).astype(np.complex128)) /
+                                   np.linalg.norm(ref.astype(np.complex128))))
+            assert r.iters == k
+    H.close()
+    mean = {f: float(np.mean(v)) for f, v in err.items()}
+    print(f"  mean error device {mean['device']:.3e} host {mean['host']:.3e}", flush=True)
+    assert mean["device"] <= mean["host"]

@@ -248,18 +248,21 @@ __global__ __launch_bounds__(64) void lz_expmv_check_kernel(double *ab, PartialN
       for (int i = mm - 1; i >= l; --i) {
         const double ei = lane_value(e, i), di = lane_value(d, i), di1 = lane_value(d, i + 1);
         const double f = s * ei, bb = c * ei;
-        const double r2 = f * f + g * g, ri = rsqrt_(r2);
-        r = r2 * ri;
-        if (!(r2 > 1e-290)) r = 0.0;   // both below 1e-145 of |T|
-        if (lane == i + 1) e = r;
-        if (r == 0.0) {
+        const double r2 = fma(f, f, g * g), ri = rsqrt_(r2);
+        // (s, c) = (f, g) / |(f, g)|, brought back to unit length by `un` = 1 - s^2 - c^2
+        // (the larger square taken off first)
+        const double s0 = f * ri, c0 = g * ri, x = fmax(fabs(s0), fabs(c0)), y = fmin(fabs(s0), fabs(c0));
+        const double un = fma(-y, y, fma(-x, x, 1.0));
+        const bool zero = !(r2 > 1e-290);   // both below 1e-145 of |T|
+        s = fma(un, 0.5 * s0, s0);
+        c = fma(un, 0.5 * c0, c0);
+        if (lane == i + 1) e = zero ? 0.0 : fma(f, s, g * c);
+        if (zero) {
           if (lane == i + 1) d -= p;
           if (lane == mm) e = 0.0;
           underflow = true;
           break;
         }
-        s = f * ri;
-        c = g * ri;
         g = di1 - p;
         r = (di - g) * s + 2.0 * c * bb;
         p = s * r;
