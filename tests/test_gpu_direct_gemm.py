@@ -108,6 +108,29 @@ def test_plan_switches_layouts(first):
     assert float(torch.linalg.vector_norm(got["bf16x6"] - out.data) / torch.linalg.vector_norm(out.data)) < 2e-6
 
 
+@pytest.mark.parametrize("prec,cplx,bar", [("bf16x6", False, 2e-6), ("fp32", False, 2e-6), ("bf16x6", True, 2e-6)])
+def test_reduced_padding_in_reused_memory(prec, cplx, bar):
+    """The reduced operands' padding is written with them: a plan whose buffers held
+    another plan's NaN gives the same bits as one on fresh buffers."""
+    print(f"[case] reused buffers {prec} {'complex' if cplx else 'real'}", flush=True)
+    eff, psi = _problem([3, 17, 29, 18, 2], 13, cplx)
+    d_eff, x = [to_device(t) for t in eff], to_device(psi)
+    bad = [to_device(t) for t in eff]
+    for t in (bad[0], bad[3]):
+        t.data.fill_(float("nan"))
+    H = EffectiveHamiltonian(d_eff, x, precision=prec)
+    want = (H @ x).data
+    num = to_oracle(H @ x, psi)
+    ref = eff_ham_mul_two_site_state(eff, psi)
+    scale = np.sqrt(sum(float((np.abs(v) ** 2).sum()) for v in ref.blocks.values()))
+    assert np.sqrt(sum(float((np.abs(num.blocks[k] - v) ** 2).sum()) for k, v in ref.blocks.items())) < bar * scale
+    del H
+    B = EffectiveHamiltonian(bad, x, precision=prec)
+    assert torch.isnan(torch.view_as_real((B @ x).data) if cplx else (B @ x).data).any()
+    B.close()
+    assert torch.equal((EffectiveHamiltonian(d_eff, x, precision=prec) @ x).data, want)
+
+
 def test_in_place_product():
     """qlg_matvec with one buffer as input and output."""
     print("[case] in place", flush=True)

@@ -32,6 +32,7 @@ Plan *build_batch_plan(Ctx *ctx, int64_t n, Plan *const *members) {
   std::vector<std::array<int64_t, NSLOTS>> base(n), rbase(n);
   int64_t vs = 0, xs = 0, ys = 0, cs = 0, ls = 0, rs = 0;
   int64_t yrs = 0, lrs = 0, rrs = 0;   // reduced form
+  std::vector<TransDesc> rred;
   p->batch_off.assign(n + 1, 0);
   for (int64_t m = 0; m < n; ++m) {
     const Plan &q = *members[m];
@@ -47,15 +48,12 @@ Plan *build_batch_plan(Ctx *ctx, int64_t n, Plan *const *members) {
     rbase[m][SLOT_Y] = yrs;
     rbase[m][SLOT_L] = lrs;
     rbase[m][SLOT_R] = rrs;
-    for (TransDesc c : q.red_l) {
-      c.src += ls;
-      c.dst += lrs;
-      p->red_l.push_back(c);
-    }
-    for (TransDesc c : q.red_r) {
-      c.src += rs;
-      c.dst += rrs;
-      p->red_r.push_back(c);
+    for (size_t k = 0; k < q.red.size(); ++k) {
+      TransDesc c = q.red[k];
+      const bool l = k < q.red_nl;
+      c.src += l ? ls : rs;
+      c.dst += l ? lrs : rrs;
+      (l ? p->red : rred).push_back(c);
     }
     yrs += q.yred_elems;
     lrs += q.lred_elems;
@@ -77,6 +75,8 @@ Plan *build_batch_plan(Ctx *ctx, int64_t n, Plan *const *members) {
   p->c_elems = cs;
   p->lint_elems = ls;
   p->rint_elems = rs;
+  p->red_nl = p->red.size();
+  p->red.insert(p->red.end(), rred.begin(), rred.end());
   p->yred_elems = yrs;
   p->lred_elems = lrs;
   p->rred_elems = rrs;

@@ -88,6 +88,7 @@ struct TransDesc {
   int64_t src, dst;
   int64_t sld, dsx;
   int32_t nz, nx;
+  int32_t pad = 0;   // zeros written after each row's nz elements (tile_trans_kernel)
 };
 
 // Split-K: a task whose K is long runs as `parts` tasks over consecutive K

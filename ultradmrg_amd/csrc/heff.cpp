@@ -307,6 +307,7 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
   };
   std::map<int, LStack> lst;
   std::vector<TransDesc> lcopy, rcopy;   // environment blocks -> FP64 form
+  std::vector<TransDesc> lred, rred;     // FP64 form -> reduced form
   int64_t lint_elems = 0, lred_elems = 0;
   auto ld8 = [](int64_t k) { return (k + 7) / 8 * 8; };
   // (unpadded where the padding alone would push an operand past the kernels' span)
@@ -332,7 +333,8 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
       for (int64_t w = 0; w < Wm; ++w) {
         const int64_t k0 = s.kbase + r0 + w * Dap;
         lcopy.push_back(TransDesc{L.off[lb] + w * Da, k0, Wm * Da, s.kld, (int32_t)Dap, (int32_t)Da});
-        p.red_l.push_back(TransDesc{k0, s.base + (r0 + w) * lda, s.kld, Wm * lda, (int32_t)Da, (int32_t)Dap});
+        lred.push_back(TransDesc{k0, s.base + (r0 + w) * lda, s.kld, Wm * lda, (int32_t)Da, (int32_t)Dap,
+                                 (int32_t)(lda - Da)});
       }
     }
     lred_elems += s.rows * lda;
@@ -416,7 +418,8 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
       const int64_t w = R.ax[1].deg[R.blk[rb][1]] * R.ax[2].deg[R.blk[rb][2]];
       const int64_t c0 = P.col[{R.blk[rb][1], R.blk[rb][2]}], k0 = P.kbase + c0 * P.kld;
       rcopy.push_back(TransDesc{R.off[rb], k0, w, P.kld, (int32_t)Dbp, (int32_t)w});
-      p.red_r.push_back(TransDesc{k0, P.base + c0, P.kld, P.ld, (int32_t)w, (int32_t)Dbp});
+      rred.push_back(TransDesc{k0, P.base + c0, P.kld, P.ld, (int32_t)w, (int32_t)Dbp,
+                               (int32_t)(c0 + w == P.K ? P.ld - P.K : 0)});
     }
     rred_elems += Dbp * P.ld;
     rint_elems += P.K * P.kld;
@@ -795,15 +798,19 @@ Plan *build_plan(Ctx *ctx, int nphys, const qlg_bsten *Ld, const qlg_bsten *cons
     check_copies(p.pack_out, p.vec.size, p.vec.size, "unpack");
     auto check_trans = [](const std::vector<TransDesc> &v, int64_t src_n, int64_t dst_n, const char *what) {
       for (const TransDesc &c : v)
-        QLG_CHECK(c.nz > 0 && c.nx > 0 && c.src >= 0 && c.dst >= 0 && c.sld >= c.nx && c.dsx >= c.nz &&
+        QLG_CHECK(c.nz > 0 && c.nx > 0 && c.src >= 0 && c.dst >= 0 && c.pad >= 0 && c.sld >= c.nx &&
+                      c.dsx >= c.nz + c.pad &&
                       c.src + (int64_t)(c.nz - 1) * c.sld + c.nx <= src_n &&
-                      c.dst + (int64_t)(c.nx - 1) * c.dsx + c.nz <= dst_n,
+                      c.dst + (int64_t)(c.nx - 1) * c.dsx + c.nz + c.pad <= dst_n,
                   std::string("copy list out of bounds: ") + what);
     };
     check_trans(lcopy, extent(L), lint_elems, "L repack");
     check_trans(rcopy, extent(R), rint_elems, "R repack");
-    check_trans(p.red_l, lint_elems, lred_elems, "L reduced form");
-    check_trans(p.red_r, rint_elems, rred_elems, "R reduced form");
+    check_trans(lred, lint_elems, lred_elems, "L reduced form");
+    check_trans(rred, rint_elems, rred_elems, "R reduced form");
+    p.red = std::move(lred);
+    p.red_nl = p.red.size();
+    p.red.insert(p.red.end(), rred.begin(), rred.end());
   }
   for (int i = 0; i < 3; ++i) {
     p.rst[i].flops = p.st[i].flops;
@@ -931,8 +938,42 @@ Plan::~Plan() {
   if (host_lz) (void)hipHostFree(host_lz);
 }
 
+namespace {
+std::mutex g_tile_mu;
+struct TileChoice {
+  int bm = 0, bn = 0;
+  bool split = false;   // split-K parts (stage 3)
+  bool operator==(const TileChoice &o) const { return bm == o.bm && bn == o.bn && split == o.split; }
+};
+std::unordered_map<std::string, TileChoice> g_tile_cache;   // signature -> tile shape and split-K
+int g_tune_hits = 0, g_tune_misses = 0;
+
+// the choice tuned for this stage's signature, if there is one (QLG_SPLITK
+// overrides what was tuned without it)
+bool cached_choice(const Stage &g, int i, int variant, TileChoice &choice) {
+  std::lock_guard<std::mutex> lk(g_tile_mu);
+  const auto it = g_tile_cache.find(tile_signature(g, i, variant));
+  if (it == g_tile_cache.end()) return false;
+  choice = it->second;
+  if (std::getenv("QLG_SPLITK")) choice.split = g.splitk;
+  return true;
+}
+
+bool autotune_enabled() {
+  static const bool on = [] {
+    const char *v = std::getenv("QLG_AUTOTUNE");
+    return !(v && v[0] == '0');
+  }();
+  return on;
+}
+}  // namespace
+
+int Plan::tile_variant() const { return precision * 2 + (dtype == QLG_C128 ? 1 : 0); }
+bool Plan::tuned() const { return !tiles_pinned && autotune_enabled() && kind == PLAN_HEFF; }
+
 // Tile lists and uploads of the form the current precision uses, on its first
-// use.
+// use: with the shapes tuned for a stage of this signature, if any were, so that
+// the first matvec neither makes nor uploads them again.
 void Plan::prepare_lists() {
   const int form = precision == QLG_PREC_F64 ? 0 : 1;
   if (lists_ready[form]) return;
@@ -940,11 +981,12 @@ void Plan::prepare_lists() {
   if (!tile_pin.empty())
     std::sscanf(tile_pin.c_str(), "%dx%d,%dx%d,%dx%d", &pinned[0][0], &pinned[0][1], &pinned[1][0], &pinned[1][1],
                        &pinned[2][0], &pinned[2][1]);
+  for (const auto &shape : pinned) tiles_pinned = tiles_pinned || shape[0] > 0;
   for (int i = 0; i < 3; ++i) {
     Stage &g = stage(i);
+    TileChoice choice;
     if (pinned[i][0] > 0) {
       g.make_tiles(pinned[i][0], pinned[i][1]);
-      tiles_pinned = true;
     } else if (i == 1) {
       // MPO stage: HBM-bound.  X is re-read once per row tile, so the row
       // tile covers K_out where the MFMA padding stays cheap; the cost counts
@@ -963,6 +1005,9 @@ void Plan::prepare_lists() {
         }
       }
       g.make_tiles(bm_best, bm_best == 64 ? 64 : 128);
+    } else if (tuned() && !g.tasks.empty() && cached_choice(g, i, tile_variant(), choice)) {
+      g.split_on = choice.split;
+      g.make_tiles(choice.bm, choice.bn);
     } else {
       model_tiles(g, dtype == QLG_C128);   // replaced by measured shapes on the first matvec
     }
@@ -1014,27 +1059,25 @@ void Plan::prepare_reduced() {
   if (planar() ? planar_ready : reduced_ready) return;
   // L stacks and R panels made from the FP64 form's, transposed: three bf16
   // piece planes each (real split-BF16, where the MPO stage writes Y as planes
-  // too), or FP32.  Padding, and Y entries that no channel writes, stay zero.
+  // too), or FP32.  Their padding, and Y entries that no channel writes, are zero.
   const int64_t ed = elem_doubles(dtype);   // complex data: (re, im) pairs of floats
   const bool pl = planar();
   const int64_t eb = pl ? 3 * 2 : ed * (int64_t)sizeof(float);   // bytes per element
   DevBuf &Lo = pl ? Lp : Lint32, &Ro = pl ? Rp : Rint32, &Yo = pl ? Yp : Y32;
-  DevBuf dl, dr;
-  auto zeroed = [&](DevBuf &buf, int64_t n) {
-    buf.ensure((size_t)(std::max<int64_t>(n, 1) * eb));
-    QLG_HIP(hipMemsetAsync(buf.p, 0, (size_t)(std::max<int64_t>(n, 1) * eb), ctx->stream));
-  };
-  auto transposed = [&](const std::vector<TransDesc> &descs, DevBuf &dd, const DevBuf &src, DevBuf &out, int64_t n) {
-    zeroed(out, n);
-    if (descs.empty()) return;
-    dd.ensure(descs.size() * sizeof(TransDesc));
-    QLG_HIP(hipMemcpyAsync(dd.p, descs.data(), descs.size() * sizeof(TransDesc), hipMemcpyHostToDevice, ctx->stream));
-    launch_tile_trans(ed == 2, pl ? 2 : 1, dd.as<TransDesc>(), (int)descs.size(), src.as<double>(), out.p, n,
+  DevBuf lists;   // one copy for both operands' lists
+  lists.ensure(std::max<size_t>(1, red.size()) * sizeof(TransDesc));
+  if (!red.empty())
+    QLG_HIP(hipMemcpyAsync(lists.p, red.data(), red.size() * sizeof(TransDesc), hipMemcpyHostToDevice, ctx->stream));
+  auto transposed = [&](size_t first, size_t count, const DevBuf &src, DevBuf &out, int64_t n) {
+    out.ensure((size_t)(std::max<int64_t>(n, 1) * eb));
+    launch_tile_trans(ed == 2, pl ? 2 : 1, lists.as<TransDesc>() + first, (int)count, src.as<double>(), out.p, n,
                       ctx->stream);
   };
-  transposed(red_l, dl, Lint, Lo, lred_elems);
-  transposed(red_r, dr, Rint, Ro, rred_elems);
-  zeroed(Yo, yred_elems);
+  transposed(0, red_nl, Lint, Lo, lred_elems);
+  transposed(red_nl, red.size() - red_nl, Rint, Ro, rred_elems);
+  const size_t y_bytes = (size_t)(std::max<int64_t>(yred_elems, 1) * eb);
+  Yo.ensure(y_bytes);
+  QLG_HIP(hipMemsetAsync(Yo.p, 0, y_bytes, ctx->stream));
   C32.ensure(std::max<int64_t>(c_elems * ed, 1) * sizeof(float));
   launch_f64_to_f32(C.as<double>(), C32.as<float>(), c_elems * ed, ctx->stream);
   (pl ? planar_ready : reduced_ready) = true;
@@ -1097,25 +1140,6 @@ void Plan::launch_stage(int i, const Slots &s) {
     launch_splitk_reduce(cplx, g.d_red.as<RedTask>(), g.d_redc.as<RedChunk>(), (int)g.redc.size(), s, stream);
 }
 
-namespace {
-std::mutex g_tile_mu;
-struct TileChoice {
-  int bm = 0, bn = 0;
-  bool split = false;   // split-K parts (stage 3)
-  bool operator==(const TileChoice &o) const { return bm == o.bm && bn == o.bn && split == o.split; }
-};
-std::unordered_map<std::string, TileChoice> g_tile_cache;   // signature -> tile shape and split-K
-int g_tune_hits = 0, g_tune_misses = 0;
-
-bool autotune_enabled() {
-  static const bool on = [] {
-    const char *v = std::getenv("QLG_AUTOTUNE");
-    return !(v && v[0] == '0');
-  }();
-  return on;
-}
-}  // namespace
-
 // Tile autotuner of the two grouped-GEMM stages.  Every tile shape (nine for
 // real FP64, seven for the real reduced modes, four for complex; the cost
 // model's ranking only orders them) is timed on
@@ -1127,9 +1151,9 @@ bool autotune_enabled() {
 void Plan::autotune(const double *in, double *out) {
   if (tuned_precision == precision) return;
   tuned_precision = precision;
-  if (tiles_pinned || !autotune_enabled() || kind != PLAN_HEFF) return;
+  if (!tuned()) return;
   const bool cplx = dtype == QLG_C128;
-  const int variant = precision * 2 + (cplx ? 1 : 0);
+  const int variant = tile_variant();
   hipStream_t stream = ctx->stream;
   const bool verbose = [] {
     const char *v = std::getenv("QLG_VERBOSE");
@@ -1138,18 +1162,11 @@ void Plan::autotune(const double *in, double *out) {
   // choices cached for this precision's shape signatures (bm = 0: not tuned yet)
   TileChoice cached[3];
   bool unchanged = step_graphs.empty() && chunk_graphs.empty();
-  {
-    std::lock_guard<std::mutex> lk(g_tile_mu);
-    for (int i : {0, 2}) {
-      const Stage &g = stage(i);
-      if (g.tasks.empty()) continue;
-      auto it = g_tile_cache.find(tile_signature(g, i, variant));
-      if (it != g_tile_cache.end()) {
-        cached[i] = it->second;
-        ++g_tune_hits;
-      }
-      if (!(cached[i] == TileChoice{g.bm, g.bn, g.split_on}) || g.tiles.empty()) unchanged = false;
-    }
+  for (int i : {0, 2}) {
+    const Stage &g = stage(i);
+    if (g.tasks.empty()) continue;
+    if (cached_choice(g, i, variant, cached[i])) ++g_tune_hits;
+    if (!(cached[i] == TileChoice{g.bm, g.bn, g.split_on}) || g.tiles.empty()) unchanged = false;
   }
   // both stages already hold the tiles chosen for this precision: nothing to
   // time or re-upload, and the stream need not drain

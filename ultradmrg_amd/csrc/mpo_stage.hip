@@ -351,15 +351,17 @@ __global__ __launch_bounds__(256) void tile_trans_kernel(const TransDesc *__rest
   if ((int)blockIdx.x >= n) return;
   const TransDesc c = d[blockIdx.x];
   const E *S = reinterpret_cast<const E *>(src) + c.src;
-  const int tz = (c.nz + 31) / 32, tx = (c.nx + 31) / 32;
+  const int nzp = c.nz + c.pad;
+  const int tz = (nzp + 31) / 32, tx = (c.nx + 31) / 32;
   const int lo = threadIdx.x & 31, hi = threadIdx.x >> 5;
   for (int i = blockIdx.y; i < tz * tx; i += kTransSplit) {
     const int z0 = i / tx * 32, x0 = i % tx * 32;
     for (int r = hi; r < 32; r += 8)
-      if (z0 + r < c.nz && x0 + lo < c.nx) t[r][lo] = S[(int64_t)(z0 + r) * c.sld + x0 + lo];
+      if (z0 + r < nzp && x0 + lo < c.nx)
+        t[r][lo] = z0 + r < c.nz ? S[(int64_t)(z0 + r) * c.sld + x0 + lo] : E{};
     __syncthreads();
     for (int r = hi; r < 32; r += 8)
-      if (x0 + r < c.nx && z0 + lo < c.nz) {
+      if (x0 + r < c.nx && z0 + lo < nzp) {
         const E v = t[lo][r];
         const int64_t o = c.dst + (int64_t)(x0 + r) * c.dsx + z0 + lo;
         if constexpr (OUT == 0) {

@@ -98,6 +98,8 @@ struct Plan {
   Stage &stage(int i) { return precision == QLG_PREC_F64 ? st[i] : rst[i]; }
   std::string tile_pin;         // QLG_TILES when the plan was built
   void prepare_lists();
+  int tile_variant() const;     // precision and data type, for the tuner's cache
+  bool tuned() const;           // whether the tuner chooses this plan's tile shapes
   DevBuf X, Y, C;
   int64_t x_elems = 0, y_elems = 0, c_elems = 0;
   int64_t vec_bytes() const;    // a vector's buffer, with one element of slack
@@ -126,7 +128,8 @@ struct Plan {
   // L stacks and R panels from Lint and Rint, and FP32 copies of the L stacks,
   // R panels and channel operators (made on first use).
   int64_t lred_elems = 0, rred_elems = 0, yred_elems = 0;
-  std::vector<TransDesc> red_l, red_r;
+  std::vector<TransDesc> red;   // L stacks' copies, then the R panels'
+  size_t red_nl = 0;            // how many of them are L's
   // T1 reuses X (stage 1 rewrites all of it every matvec); Y32 is a buffer of
   // its own because stage 3 reads Y entries that no channel writes, which must
   // stay zero.
