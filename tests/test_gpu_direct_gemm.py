@@ -158,3 +158,19 @@ def test_batch_in_split_mode():
         B.matvec_into(x, y)
         for (eff, psi), got in zip(probs, B.unpack(y)):
             assert _err(got, eff_ham_mul_two_site_state(eff, psi)) < bar
+
+
+def test_batch_keeps_pinned_tiles(monkeypatch):
+    """QLG_TILES holds for the batch of pinned plans too: the same tiles, so the same
+    bits as the members' own products."""
+    print("[case] pinned batch", flush=True)
+    monkeypatch.setenv("QLG_TILES", "32x32,64x64,128x128")
+    probs = [_problem(d, s) for s, d in enumerate(([30, 170, 290, 160, 20], [10, 140, 133, 9]))]
+    members = [EffectiveHamiltonian([to_device(t) for t in eff], to_device(psi)) for eff, psi in probs]
+    B = BatchedEffectiveHamiltonian(members)
+    x = B.pack([to_device(psi) for _, psi in probs])
+    y = torch.empty_like(x)
+    torch.cuda.synchronize()
+    B.matvec_into(x, y)
+    for m, (_, psi), got in zip(members, probs, B.unpack(y)):
+        assert torch.equal((m @ to_device(psi)).data, got.data)

@@ -28,6 +28,7 @@ Plan *build_batch_plan(Ctx *ctx, int64_t n, Plan *const *members) {
   p->dtype = dtype;
   p->precision = QLG_PREC_F64;
   p->nphys = members[0]->nphys;
+  p->tile_pin = members[0]->tile_pin;
   // arena bases of every member, per slot
   std::vector<std::array<int64_t, NSLOTS>> base(n), rbase(n);
   int64_t vs = 0, xs = 0, ys = 0, cs = 0, ls = 0, rs = 0;
