@@ -71,6 +71,18 @@ def test_edge_sectors(monkeypatch, degs, cplx, shape):
     assert _err(H @ to_device(psi), ref) < 1e-12
 
 
+@pytest.mark.parametrize("cplx,shape", [(False, s) for s in ("32x32", "64x32", "32x64", "64x64", "128x64", "64x128",
+                                                             "128x128", "64x16", "128x16")] +
+                         [(True, s) for s in ("32x32", "64x32", "32x64", "64x64")])
+@pytest.mark.parametrize("degs", [EDGES, LONG], ids=["edges", "long"])
+def test_edge_sectors_lds_kernel(monkeypatch, degs, cplx, shape):
+    """The same on the LDS-staged kernel, which serves the plans whose spans the
+    direct one cannot address (QLG_DIRECT=0 puts any plan there)."""
+    print(f"[case] LDS kernel {degs} {'complex' if cplx else 'real'} {shape}", flush=True)
+    monkeypatch.setenv("QLG_DIRECT", "0")
+    test_edge_sectors(monkeypatch, degs, cplx, shape)
+
+
 @pytest.mark.parametrize("shape", ["128x64", "64x128", "128x128"])
 @pytest.mark.parametrize("degs", [EDGES, LONG], ids=["edges", "long"])
 def test_wide_complex_tiles(monkeypatch, degs, shape):

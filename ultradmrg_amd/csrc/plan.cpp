@@ -286,10 +286,13 @@ void make_tiles_lpt(std::vector<GemmTile> &tiles, const std::vector<std::array<i
 // [K x N], unconjugated.  Real data is read in pairs that may reach one element
 // past an operand's last row, so its operands must be the plan's own (padded
 // panels, vectors with slack).  A slice's scalar offset reaches up to 15 rows
-// past K and has to stay below 2^31 bytes.  Other stages (the contractions
-// around the solve) run on the LDS kernel.
+// past K and has to stay below 2^31 bytes: real operands get there only with
+// rows of 2^23 elements, complex ones only in the last 16 rows below the span
+// that validate_stage allows.  Those stages run on the LDS kernel, as do the
+// contractions around the solve.  QLG_DIRECT=0 sends every stage there.
 void Stage::find_direct() {
   direct = false;
+  if (const char *v = std::getenv("QLG_DIRECT"); v && v[0] == '0') return;
   for (const GemmTask &t : tasks)
     for (int q = 0; q < t.seg_count; ++q) {
       const GemmSeg &g = segs[t.seg_begin + q];
@@ -489,7 +492,7 @@ std::string tile_signature(const Stage &s, int stage, int variant) {
       best = c.second;
       top = c.first;
     }
-  return std::to_string(stage) + "/" + std::to_string(variant) + "/" +
+  return std::to_string(stage) + "/" + std::to_string(variant) + (s.direct ? "d/" : "/") +
          std::to_string(tot > 0 ? (int)std::lround(std::log2(tot)) : -1) + "/" + std::to_string(top);
 }
 
