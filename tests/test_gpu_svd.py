@@ -138,3 +138,36 @@ def test_block_svd_degenerate_gram(cplx):
     rec = contract(contract(r.u, r.s, 1), r.vt, 1).blocks()
     for k, b in blocks.items():
         assert np.abs(rec.get(k, np.zeros_like(b)) - b).max() < 1e-10
+
+
+@pytest.mark.parametrize("rows", [(1, 2, 5), (28, 16, 17, 1), (29, 16, 17, 1), (28, 27, 3, 90), (32, 31, 33)],
+                         ids=["few", "28", "29", "28+90", "32+33"])
+@pytest.mark.parametrize("decades", [5, 13])
+def test_block_svd_at_the_small_solver_limit(rows, decades):
+    """Real calls on both sides of the rule that sends them to the in-LDS eigensolver
+    (every sector has at most 28 rows), both orientations of each size.  Values vs
+    numpy to 1e-12 of the largest, orthonormal u and vt; what is kept down to 1e-5
+    of a sector's largest reconstructs to 1e-10 (eps s_max^2 / s_min is 2e-11)."""
+    print(f"[case] library block svd rows {rows} decades {decades}", flush=True)
+    rng = np.random.default_rng(sum(rows) + decades)
+    dims = [d for n in rows for d in ((n, n + 7), (n + 12, n))]
+    a_ax = Axis.make([((2 * i,), r) for i, (r, _) in enumerate(dims)], -1)
+    b_ax = Axis.make([((2 * i,), c) for i, (_, c) in enumerate(dims)], 1)
+    blocks = {}
+    for i, (r, c) in enumerate(dims):
+        n = min(r, c)
+        blocks[(i, i)] = (_orth(rng, r, n, False) * np.logspace(0, -decades, n) * 2.0 ** -i) @ _orth(rng, c, n, False).T
+    spectra = [np.linalg.svd(blocks[(i, i)], compute_uv=False) for i in range(len(dims))]
+    r = block_svd(BlockTensor.from_blocks([a_ax, b_ax], blocks), 1, (0,), 0.0, 10 ** 6, 10 ** 6)
+    assert r.D == sum(map(len, spectra))
+    for (mi, _), blk in r.s.blocks().items():
+        got, ref = np.diag(blk), spectra[r.u.axes[-1].qns[mi][0] // 2]
+        assert np.abs(got - ref[:len(got)]).max() <= 1e-12
+    for (i, mi), U in r.u.blocks().items():
+        assert np.abs(U.T @ U - np.eye(U.shape[1])).max() < 1e-12
+    for (mi, j), V in r.vt.blocks().items():
+        assert np.abs(V @ V.T - np.eye(V.shape[0])).max() < 1e-12
+    if decades <= 5:
+        rec = contract(contract(r.u, r.s, 1), r.vt, 1).blocks()
+        for k, b in blocks.items():
+            assert np.abs(rec[k] - b).max() < 1e-10
