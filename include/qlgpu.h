@@ -341,7 +341,8 @@ int qlg_svd_destroy(qlg_svd r);
  * eigenvalues in ascending order.  Real groups of order 32 and less: cyclic
  * Jacobi in LDS; all others: divide and conquer.  Groups run concurrently.  The
  * call returns after the work is complete (it checks the solver's convergence
- * flags); QLG_ERR_NUMERIC if a matrix did not converge. */
+ * flags); QLG_ERR_NUMERIC if a matrix did not converge.  A real matrix of
+ * order 32 or less with an element that is not finite comes back as NaN. */
 typedef struct {
   int64_t n;      /* order of each matrix   */
   int64_t batch;  /* matrices in the group  */

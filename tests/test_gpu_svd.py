@@ -17,6 +17,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
+    from ultradmrg_amd._lib import QlgError
     from ultradmrg_amd.sweep import block_svd
     from ultradmrg_amd.tensor import Axis, BlockTensor, contract
 
@@ -171,3 +172,18 @@ def test_block_svd_at_the_small_solver_limit(rows, decades):
         rec = contract(contract(r.u, r.s, 1), r.vt, 1).blocks()
         for k, b in blocks.items():
             assert np.abs(rec[k] - b).max() < 1e-10
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_block_svd_refuses_non_finite(bad):
+    """One element that is not finite in a call of small sectors is an error, not a
+    state of zeros."""
+    print(f"[case] library block svd with {bad}", flush=True)
+    rng = np.random.default_rng(0)
+    dims = [(12, 15), (20, 9)]
+    a_ax = Axis.make([((2 * i,), r) for i, (r, _) in enumerate(dims)], -1)
+    b_ax = Axis.make([((2 * i,), c) for i, (_, c) in enumerate(dims)], 1)
+    blocks = {(i, i): rng.standard_normal(d) for i, d in enumerate(dims)}
+    blocks[(0, 0)][4, 5] = bad
+    with pytest.raises(QlgError, match="not finite"):
+        block_svd(BlockTensor.from_blocks([a_ax, b_ax], blocks), 1, (0,), 1e-10, 1, 100)

@@ -493,6 +493,11 @@ SvdResult *block_svd(Ctx &c, const qlg_bsten *desc, int ldims, const int32_t *ld
   std::vector<double> hsv, hscale;
   download<double>(c, hscale, scale.p, xm.size());
   download<double>(c, hsv, sv.p, (size_t)nsv);
+  // the in-LDS solver passes a NaN or an infinity through as NaN and reports no
+  // failure, so they are looked for here
+  if (small)
+    for (double v : hsv)
+      if (!std::isfinite(v)) throw Error(QLG_ERR_NUMERIC, "block SVD: the tensor has an element that is not finite");
 
   // ---- cluster refinement: sectors whose kept values reach below 1e-6 of their largest --
   // (decided on the first values; the refined values then decide the truncation)
