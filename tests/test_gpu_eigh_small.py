@@ -111,3 +111,27 @@ def test_upper_triangle_is_the_input():
     half = eigh_batched([torch.from_numpy(np.triu(g) + np.tril(np.full(g.shape, 7.5), -1)).cuda() for g in groups])
     for (w, v), (wh, vh) in zip(whole, half):
         assert torch.equal(w, wh) and torch.equal(v, vh)
+
+
+@pytest.mark.parametrize("n", [16, 24, 32])
+def test_no_less_accurate_than_the_library(n):
+    """Residual and orthonormality of the in-LDS solver, means over 24 random and 24
+    graded matrices in extended precision, against the library's solver on the same
+    matrices as complex ones.  Both are orthogonal methods whose mean errors are
+    those of many roundings; a quarter is allowed for the means' scatter."""
+    print(f"[case] accuracy at order {n}", flush=True)
+    rng = np.random.default_rng(100 + n)
+    mats = [_matrix(k, n, rng) for k in ("random", "graded") for _ in range(24)]
+    mats = np.stack([(a + a.T) / 2 for a in mats])
+    err = {}
+    for name, dt in (("small", np.float64), ("library", np.complex128)):
+        (w, v), = eigh_batched([torch.from_numpy(mats.astype(dt)).cuda()])
+        w, v = w.cpu().numpy().astype(np.longdouble), v.cpu().numpy().astype(np.clongdouble)
+        res = [np.linalg.norm((a @ vi - vi * wi).astype(complex)) / np.linalg.norm(a, 2)
+               for a, wi, vi in zip(mats, w, v)]
+        orth = [np.linalg.norm((vi.conj().T @ vi - np.eye(n)).astype(complex)) for vi in v]
+        err[name] = np.mean(res), np.mean(orth)
+    print(f"  residual {err['small'][0]:.2e} library {err['library'][0]:.2e}, orthonormality "
+          f"{err['small'][1]:.2e} library {err['library'][1]:.2e}", flush=True)
+    assert err["small"][0] <= 1.25 * err["library"][0]
+    assert err["small"][1] <= 1.25 * err["library"][1]
