@@ -327,8 +327,9 @@ static void launch_shape(int bm, int bn, int bk, const GemmTile *tiles, const Ge
 // (5.6 GFLOP each) stage 1 177 -> 145 us, stage 3 188 (and 17 for split-K's
 // reduce) -> 137 us; dense 8 x (4096 x 4096 x 2048) 72 TFLOP/s.  The two-waves
 // launch bound keeps the accumulators in vector registers: without it each
-// slice moved them to and from the accumulation registers.  What is left is
-// padding to 16-wide blocks, the last wave of tiles and the stores of T1.
+// slice moved them to and from the accumulation registers.  Counters of the
+// two: MFMA pipe busy 0.56 and 0.65, waiting on memory 0.22 and 0.11 of the wave
+// cycles, 1.7 and 3.0 waves per SIMD, padding to 16-wide blocks 1.10 and 1.19.
 // ---------------------------------------------------------------------------
 __device__ inline double2 load_pair(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   typedef double d2 __attribute__((ext_vector_type(2)));

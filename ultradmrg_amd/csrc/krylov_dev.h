@@ -31,7 +31,7 @@ void lz_gs_check(hipStream_t st, double *ab, PartialNorm norm, LzCtl *ctl, int m
 // Iteration m of LanczosExpmvSolver: coef_cur <- exp(-i tau T_{m+1}) e_1
 // (interleaved complex, zero beyond m), its Distance to coef_prev, the stop
 // rule of lanczos_expmv_solver_impl.h:162-167 (plus breakdown); coef_prev
-// takes coef_cur when the solve goes on.  z: workspace of kMaxExpmvDim^2 doubles.
+// takes coef_cur when the solve goes on.  norm as in lz_gs_check.
 void lz_expmv_check(hipStream_t st, double *ab, PartialNorm norm, LzCtl *ctl, double *coef_cur, double *coef_prev,
                     int m, int64_t dim, int64_t maxit, double err, double tau);
 // Classical Gram-Schmidt of g against bases[0..k): c = V^H g, g <- g - V c,

@@ -51,6 +51,10 @@ __global__ void lz_reset_kernel(LzCtl *ctl) {
 // their divisions and square roots: these come from the hardware estimates and
 // two Newton steps (within an ulp or two), a third of the IEEE sequences'
 // latency.  Arguments stay far from the range's ends (see the callers).
+// Against 113-bit arithmetic that costs the bisected eigenvalue nothing (mean
+// error 8.6e-17 |T| at order 6, 8.5e-17 with divisions, equal from order 16);
+// the QL rotations are brought back to unit length, which leaves the
+// exponential's coefficients at 3.3e-16 where divisions give 4.3e-16.
 __device__ inline double recip(double x) {
   double r = __builtin_amdgcn_rcp(x);
   r = fma(fma(-x, r, 1.0), r, r);
