@@ -36,3 +36,15 @@ def test_given_offsets_and_short_buffers():
         BlockTensor._on_layout([A, B], [(0, 0)], [0], 6, torch.zeros(5))
     with pytest.raises(IndexError):
         BlockTensor([A, B], [(3, 0)], torch.zeros(40))
+
+
+@pytest.mark.parametrize("offsets", [[20, 0], (20, 0), np.array([20, 0]), torch.tensor([20, 0]), iter([20, 0])],
+                         ids=["list", "tuple", "array", "tensor", "iterator"])
+def test_forms_of_offsets(offsets):
+    t = BlockTensor([A, B], (iter(c) for c in ((0, 0), (2, 1))), torch.zeros(40), offsets)
+    assert t.coords == [(0, 0), (2, 1)] and t.offsets == [20, 0] and t.size == 26
+
+
+def test_uneven_coordinates_stay_as_given():
+    t = BlockTensor([A, B], [(0, 1, 1), (0,)], torch.zeros(40))
+    assert t.coords == [(0, 1, 1), (0,)] and t.offsets == [0, 15] and t.size == 18

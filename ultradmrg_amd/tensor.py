@@ -61,16 +61,18 @@ class BlockTensor:
         self.axes = list(axes)
         # whole-array bookkeeping: a two-site tensor has hundreds of blocks, and a
         # Python loop over them costs more than the contraction that made it
-        coords = list(coords)
-        ints = np.fromiter(chain.from_iterable(coords), dtype=np.int64)
-        ints = ints.reshape(len(coords), -1 if coords else len(self.axes))
-        self.coords = list(map(tuple, ints.tolist()))
-        sizes = np.ones(len(ints), dtype=np.int64)
-        for ax, col in zip(self.axes, ints.T):
-            sizes *= np.array(ax.degs, dtype=np.int64)[col]
-        if offsets is None:
-            offsets = np.cumsum(sizes) - sizes
-        offs = np.array(offsets, dtype=np.int64).reshape(-1)
+        coords = list(map(tuple, coords))
+        if len(set(map(len, coords))) > 1:   # no array: as given
+            self.coords = [tuple(int(v) for v in c) for c in coords]
+            sizes = np.array([self.block_size(c) for c in self.coords], dtype=np.int64)
+        else:
+            ints = np.fromiter(chain.from_iterable(coords), dtype=np.int64)
+            ints = ints.reshape(len(coords), -1 if coords else len(self.axes))
+            self.coords = list(map(tuple, ints.tolist()))
+            sizes = np.ones(len(ints), dtype=np.int64)
+            for ax, col in zip(self.axes, ints.T):
+                sizes *= np.array(ax.degs, dtype=np.int64)[col]
+        offs = np.cumsum(sizes) - sizes if offsets is None else np.fromiter(offsets, dtype=np.int64)
         self.offsets = offs.tolist()
         n = min(len(offs), len(sizes))
         self.size = int((offs[:n] + sizes[:n]).max()) if n else 0
